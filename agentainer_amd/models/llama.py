@@ -98,6 +98,9 @@ class LlamaAttention(torch.nn.Module):
         # opt-in quantized decode weights ("turbo": engine.dense_quant)
         self.qkv_q = None
         self.o_q = None
+        # the model's weights are quantized (also those outside attention):
+        # decode attention sums in its fixed order
+        self.fixed_decode = False
 
     def attend(self, qkv, k_cache, v_cache, md: AttnMetadata, cos_sin,
                packed=False):
@@ -121,6 +124,12 @@ class LlamaAttention(torch.nn.Module):
                                         md.seq_lens, md.query_starts,
                                         md.query_lens, self.scale,
                                         max_qlen=md.max_qlen, packed=packed)
+        elif self.fixed_decode:
+            ops.rope_append(q, k, v, k_cache, v_cache, cos_sin, md.positions,
+                            md.slot_mapping)
+            ops.paged_decode_attention_fixed(out, q, k_cache, v_cache,
+                                             md.page_table, md.seq_lens,
+                                             self.scale)
         else:
             ops.rope_append_decode(out, q, k, v, k_cache, v_cache, cos_sin,
                                    md.positions, md.slot_mapping,
@@ -130,12 +139,9 @@ class LlamaAttention(torch.nn.Module):
 
     def stream_weights(self):
         """What forward_packed multiplies, or None where it cannot run."""
-        qkv = self.qkv_packed if self.qkv_q is None else self.qkv_q
-        o = self.o_packed if self.o_q is None else self.o_q
-        if (qkv is None or o is None
-                or self.cfg.hidden_size % ops.stream_k(qkv)):
+        if self.qkv_packed is None or self.o_packed is None:
             return None
-        return qkv, o
+        return self.qkv_packed, self.o_packed
 
     def forward_packed(self, x, T, k_cache, v_cache, md, cos_sin):
         """Packed rows in (row-major above ops.STREAM_ROWS, where the fused
@@ -186,13 +192,10 @@ class LlamaMLP(torch.nn.Module):
 
     def stream_weights(self):
         """What forward_packed multiplies, or None where it cannot run."""
-        gate_up = (self.gate_up_packed if self.gate_up_q is None
-                   else self.gate_up_q)
-        down = self.down_packed if self.down_q is None else self.down_q
-        if (gate_up is None or down is None or self.inter % 32
-                or self.inter % ops.stream_k(down)):
+        if (self.gate_up_packed is None or self.down_packed is None
+                or self.inter % 32):
             return None
-        return gate_up, down
+        return self.gate_up_packed, self.down_packed
 
     def forward_packed(self, x, T):
         """Packed rows in, fp32 parts of the residual update out."""
@@ -245,22 +248,17 @@ class LlamaLayer(torch.nn.Module):
 
     def streams(self, T):
         """Whether forward_packed can take T rows."""
-        attn, mlp = self.attn.stream_weights(), self.mlp.stream_weights()
-        if attn is None or mlp is None:
-            return False
-        return (T <= ops.STREAM_ROWS
-                or all(isinstance(w, torch.Tensor) for w in attn + mlp))
+        return (self.attn.stream_weights() is not None
+                and self.mlp.stream_weights() is not None)
 
     def forward_packed(self, parts, residual, k_cache, v_cache, md, cos_sin):
-        """At most ops.STREAM_ROWS_BF16 rows: `parts` (None in the first layer) is
+        """At most ops.STREAM_ROWS_WIDE rows: `parts` (None in the first layer) is
         what the layer before still has to add to the residual."""
         T = residual.size(0)
         x = ops.add_parts_rmsnorm(residual, parts, self.input_ln, self.eps,
-                                  packed=T <= ops.STREAM_ROWS,
-                                  for_weight=self.attn.stream_weights()[0])
+                                  packed=T <= ops.STREAM_ROWS)
         parts = self.attn.forward_packed(x, T, k_cache, v_cache, md, cos_sin)
-        x = ops.add_parts_rmsnorm(residual, parts, self.post_ln, self.eps,
-                                  for_weight=self.mlp.stream_weights()[0])
+        x = ops.add_parts_rmsnorm(residual, parts, self.post_ln, self.eps)
         return self.mlp.forward_packed(x, T)
 
 
@@ -278,7 +276,7 @@ def forward_streamed(model, input_ids, md, kv_caches, last_rows):
     if last_rows is not None:
         x = x[last_rows]
         T = x.size(0)
-        if T > ops.STREAM_ROWS_BF16:
+        if T > ops.STREAM_ROWS_WIDE:
             return ops.linear(x, model.lm_head, model.lm_head_packed)
         x = ops.pack_rows(x)
     return ops.stream_linear(x, T, model.lm_head_packed,
@@ -286,9 +284,11 @@ def forward_streamed(model, input_ids, md, kv_caches, last_rows):
 
 
 def can_stream(model, input_ids) -> bool:
-    """Few rows, on a single-rank GPU model whose decode weights are packed."""
+    """Few rows, on a single-rank GPU model whose decode weights are packed.
+    Quantized weights are not: they keep the row-major projections and their
+    order of sums (see decode_attn_fixed.hip for what another order does)."""
     T = input_ids.numel()
-    return (input_ids.is_cuda and 0 < T <= ops.STREAM_ROWS_BF16
+    return (input_ids.is_cuda and 0 < T <= ops.STREAM_ROWS_WIDE
             and model.tp_group is None
             and getattr(model, "lm_head_packed", None) is not None
             and model.lm_head.size(0) % 32 == 0
@@ -366,6 +366,7 @@ class LlamaForCausalLM(torch.nn.Module):
         (per-channel e4m3), or "mxfp4" (e2m1 + e8m0 block-32 scales) —
         opt-in reduced-precision DECODE projections (prefill stays bf16)."""
         for layer in self.layers:
+            layer.attn.fixed_decode = bool(dense_quant)
             if dense_quant == "mxfp4":
                 for mod_, wname, qname in (
                         (layer.attn, "qkv_proj", "qkv_q"),

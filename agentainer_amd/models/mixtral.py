@@ -10,9 +10,10 @@ MoE execution model, chosen for the MI355X serving regime:
     projection covers all experts; a workgroup lists the rows its expert
     was chosen for on the device, so unchosen experts are not read and
     the step stays free of host syncs (hipGraph-capturable).
-  * Decode under EP: DENSE-ROUTED — every local expert runs on the
-    whole batch, scaled by the router's top-k-masked weight (0 for
-    unrouted tokens); same device-side control, no gather.
+  * Decode under EP or with quantized experts: DENSE-ROUTED — every
+    local expert runs on the whole batch, scaled by the router's
+    top-k-masked weight (0 for unrouted tokens); same device-side
+    control, no gather.
   * Expert parallelism (EP over RCCL/xGMI): experts are PARTITIONED
     across ranks. Decode keeps activations replicated (the attention
     all-reduce already paid for that), each rank computes its local
@@ -111,14 +112,6 @@ class MixtralMoE(torch.nn.Module):
                 or T > ops.STREAM_ROWS
                 or T * self.top_k > ops.STREAM_PAIRS or self.inter % 32):
             return None
-        for kind, gu, dn in (("mxfp4", self.gate_up_fp4, self.down_fp4),
-                             ("fp8", self.gate_up_fp8, self.down_fp8)):
-            if gu[0] is not None:
-                hid = self.cfg.hidden_size
-                gu = [(kind, w, sc, 2 * self.inter) for w, sc in gu]
-                dn = [(kind, w, sc, hid) for w, sc in dn]
-                k = ops.stream_k(gu[0])
-                return None if hid % k or self.inter % k else (gu, dn)
         if self.gate_up_packed[0] is None:
             return None
         return self.gate_up_packed, self.down_packed
@@ -415,6 +408,7 @@ class MixtralForCausalLM(torch.nn.Module):
     def pack_decode_weights(self, expert_fp8: bool = False,
                             expert_fp4: bool = False):
         for layer in self.layers:
+            layer.attn.fixed_decode = expert_fp8 or expert_fp4
             layer.attn.qkv_packed = ops.pack_weight(layer.attn.qkv_proj.data)
             layer.attn.o_packed = ops.pack_weight(layer.attn.o_proj.data)
             for i in range(layer.moe.n_local):

@@ -149,6 +149,21 @@ def paged_decode_attention(out, q, k_cache, v_cache, page_table, seq_lens,
     return out
 
 
+def paged_decode_attention_fixed(out, q, k_cache, v_cache, page_table,
+                                 seq_lens, scale: float):
+    """paged_decode_attention in an order of sums that depends on a sequence's
+    length alone, with queries requantized for fp8 pools: what decode steps of
+    models with quantized weights take (see decode_attn_fixed.hip)."""
+    mod = _dispatch("paged_decode_attention_fixed", q)
+    if mod:
+        mod.paged_decode_attention_fixed(out, q, k_cache, v_cache, page_table,
+                                         seq_lens, float(scale))
+    else:
+        reference.paged_decode_attention(out, q, k_cache, v_cache, page_table,
+                                         seq_lens, scale)
+    return out
+
+
 def paged_prefill_attention(out, q, k_cache, v_cache, page_table, seq_lens,
                             query_starts, query_lens, scale: float,
                             max_qlen: int = 0, packed: bool = False):
@@ -277,12 +292,12 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 # from every workgroup. Projections into the residual stream return fp32
 # partial sums [splits, T, N] that add_parts_rmsnorm adds up.
 
-STREAM_ROWS = 64         # any weight
-STREAM_ROWS_BF16 = 128   # pack_weight weights
+STREAM_ROWS = 64         # every projection of a layer, and experts
+STREAM_ROWS_WIDE = 128   # projections with many column tiles
 
 
 def packed_rows(T: int, K: int, device) -> torch.Tensor:
-    """Buffer for T packed rows of K columns (T <= STREAM_ROWS_BF16)."""
+    """Buffer for T packed rows of K columns (T <= STREAM_ROWS_WIDE)."""
     groups = 1
     while groups * 16 < T:
         groups *= 2
@@ -296,92 +311,43 @@ def pack_rows(x: torch.Tensor) -> torch.Tensor:
 
 
 def add_parts_rmsnorm(residual: torch.Tensor, parts: Optional[torch.Tensor],
-                      w: torch.Tensor, eps: float, packed: bool = True,
-                      for_weight=None):
+                      w: torch.Tensor, eps: float, packed: bool = True):
     """residual [T, H] += sum of parts [S, T, H] (None: nothing to add);
-    returns the RMS norm of the new residual, row-major or packed for the
-    streaming projection with weight `for_weight` (see _stream_rows)."""
+    returns the RMS norm of the new residual, row-major or packed."""
     T, H = residual.shape
-    kind = 0 if for_weight is None else _stream_weight(for_weight)[0]
-    if kind:
-        rows = _code_rows(packed_rows(T, H, residual.device), kind, T)
-        out, scale = rows
-    else:
-        out = rows = (packed_rows(T, H, residual.device) if packed
-                      else torch.empty_like(residual))
-        scale = out
+    out = (packed_rows(T, H, residual.device) if packed
+           else torch.empty_like(residual))
     _dispatch("add_parts_rmsnorm", residual).add_parts_rmsnorm(
-        out, scale, residual, parts, w, float(eps), packed, kind)
-    return rows
+        out, residual, parts, w, float(eps), packed)
+    return out
 
 
-_STREAM_KINDS = {"fp8": 1, "mxfp4": 2}
 STREAM_EXPERTS = 16   # experts of one launch
 STREAM_PAIRS = 128    # (token, choice) pairs of one launch
 
 
-def _stream_weight(w):
-    """(kind, weight, scales) of a pack_weight tensor or of a quantized
-    ("fp8" | "mxfp4", packed, scales, N) tuple."""
-    if isinstance(w, torch.Tensor):
-        return 0, w, w
-    return _STREAM_KINDS[w[0]], w[1], w[2]
-
-
-def stream_k(w) -> int:
-    """K has to be a multiple of this for a projection with weight w."""
-    return 128 if not isinstance(w, torch.Tensor) and w[0] == "mxfp4" else 32
-
-
-def _code_rows(x: torch.Tensor, kind: int, rows: int):
-    """Buffers for the codes and scales of as many packed rows as x has."""
-    return (torch.empty(x.numel() // (1 if kind == 1 else 2),
-                        dtype=torch.uint8, device=x.device),
-            torch.empty(rows, dtype=torch.float32, device=x.device))
-
-
-def _stream_rows(mod, x, kind: int, rows: int, K: int):
-    """Packed rows in the kind its weight multiplies, and their scales: x is
-    either packed bf16 rows or already (codes, scales)."""
-    if isinstance(x, tuple):
-        return x
-    if kind == 0:
-        return x, x
-    xq, scale = _code_rows(x, kind, rows)
-    mod.quant_packed(xq, scale, x, kind, rows, K)
-    return xq, scale
-
-
 def _stream(out, x, T, w, N, K, mode, split=1):
-    mod = _dispatch("stream_gemm", out)
-    kind, wq, ws = _stream_weight(w)
-    xq, xs = _stream_rows(mod, x, kind, T, K)
-    mod.stream_gemm(out, xq, xs, wq, ws, kind, T, N, K, mode, split)
+    _dispatch("stream_gemm", out).stream_gemm(out, x, w, T, N, K, mode, split)
     return out
-
-
-def _rows_device(x):
-    return (x[0] if isinstance(x, tuple) else x).device
 
 
 def stream_linear(x, T: int, w, N: int, K: int) -> torch.Tensor:
     """bf16 [T, N] = packed rows x @ W^T."""
-    out = torch.empty(T, N, dtype=torch.bfloat16, device=_rows_device(x))
+    out = torch.empty(T, N, dtype=torch.bfloat16, device=x.device)
     return _stream(out, x, T, w, N, K, 0)
 
 
 def stream_parts(x, T: int, w, N: int, K: int) -> torch.Tensor:
     """fp32 parts [S, T, N] of packed rows x @ W^T."""
     split = _load_hip().stream_splits(T, N, K)
-    out = torch.empty(split, T, N, dtype=torch.float32,
-                      device=_rows_device(x))
+    out = torch.empty(split, T, N, dtype=torch.float32, device=x.device)
     return _stream(out, x, T, w, N, K, 1, split)
 
 
 def stream_gate_up(x, T: int, w, N: int, K: int) -> torch.Tensor:
     """Packed rows of N / 2 columns: silu(x @ gate^T) * (x @ up^T) with the
     weight [gate; up]."""
-    return _stream(packed_rows(T, N // 2, _rows_device(x)), x, T, w, N, K, 2)
+    return _stream(packed_rows(T, N // 2, x.device), x, T, w, N, K, 2)
 
 
 def route_packed(x: torch.Tensor, T: int, router: torch.Tensor, top_k: int):
@@ -400,20 +366,13 @@ def stream_experts(x: torch.Tensor, T: int, choice, weight, gate_up, down,
     most STREAM_PAIRS."""
     mod = _dispatch("stream_gemm_experts", x)
     top_k = choice.size(1)
-    pairs = T * top_k
-    gu = [_stream_weight(w) for w in gate_up]
-    dn = [_stream_weight(w) for w in down]
-    xq, xs = _stream_rows(mod, x, gu[0][0], T, hidden)
-    act = torch.empty((pairs + 15) // 16 * 16 * inter, dtype=torch.bfloat16,
-                      device=x.device)
-    mod.stream_gemm_experts(act, xq, xs, [w[1] for w in gu],
-                            [w[2] for w in gu], gu[0][0], choice, weight,
-                            2 * inter, hidden, 2)
-    aq, asc = _stream_rows(mod, act, dn[0][0], pairs, inter)
+    act = torch.empty((T * top_k + 15) // 16 * 16 * inter,
+                      dtype=torch.bfloat16, device=x.device)
+    mod.stream_gemm_experts(act, x, list(gate_up), choice, weight, 2 * inter,
+                            hidden, 2)
     out = torch.empty(top_k, T, hidden, dtype=torch.float32, device=x.device)
-    mod.stream_gemm_experts(out, aq, asc, [w[1] for w in dn],
-                            [w[2] for w in dn], dn[0][0], choice, weight,
-                            hidden, inter, 1)
+    mod.stream_gemm_experts(out, act, list(down), choice, weight, hidden,
+                            inter, 1)
     return out
 
 

@@ -83,6 +83,7 @@ SOURCES = [
     "rope.hip",
     "kvcache.hip",
     "decode_attn.hip",
+    "decode_attn_fixed.hip",
     "prefill_attn.hip",
     "sampling.hip",
     "skinny_gemm.hip",

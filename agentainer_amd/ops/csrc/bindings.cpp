@@ -23,6 +23,10 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor page_table, torch::Tensor seq_lens,
                             double scale);
+void paged_decode_attention_fixed(torch::Tensor out, torch::Tensor q,
+                                  torch::Tensor k_cache, torch::Tensor v_cache,
+                                  torch::Tensor page_table,
+                                  torch::Tensor seq_lens, double scale);
 void paged_prefill_attention(torch::Tensor out, torch::Tensor q,
                              torch::Tensor k_cache, torch::Tensor v_cache,
                              torch::Tensor page_table, torch::Tensor seq_lens,
@@ -46,23 +50,17 @@ void skinny_gemm_mxfp4(torch::Tensor out, torch::Tensor x8, torch::Tensor sx,
 void skinny_gemm_fp8(torch::Tensor out, torch::Tensor x8, torch::Tensor sx,
                      torch::Tensor w_packed, torch::Tensor sw, long N, long K,
                      torch::Tensor ws, long split);
-void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor x_scale,
-                 torch::Tensor w, torch::Tensor w_scale, long kind, long M,
+void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w, long M,
                  long N, long K, long mode, long split);
 void stream_gemm_experts(torch::Tensor out, torch::Tensor x,
-                         torch::Tensor x_scale, std::vector<torch::Tensor> w,
-                         std::vector<torch::Tensor> w_scale, long kind,
-                         torch::Tensor choice, torch::Tensor weight, long N,
-                         long K, long mode);
-void quant_packed(torch::Tensor xq, torch::Tensor scale, torch::Tensor x,
-                  long kind, long rows, long K);
+                         std::vector<torch::Tensor> w, torch::Tensor choice,
+                         torch::Tensor weight, long N, long K, long mode);
 void route_packed(torch::Tensor choice, torch::Tensor weight, torch::Tensor x,
                   torch::Tensor router);
 long stream_splits(long M, long N, long K);
-void add_parts_rmsnorm(torch::Tensor out, torch::Tensor out_scale,
-                       torch::Tensor residual,
+void add_parts_rmsnorm(torch::Tensor out, torch::Tensor residual,
                        c10::optional<torch::Tensor> parts, torch::Tensor w,
-                       double eps, bool packed, long kind);
+                       double eps, bool packed);
 void pack_rows(torch::Tensor out, torch::Tensor x);
 void route_rows(torch::Tensor choice, torch::Tensor weight, torch::Tensor order,
                 torch::Tensor place, torch::Tensor counts, torch::Tensor x,
@@ -87,6 +85,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append, "scatter new k/v into the paged KV cache");
   m.def("paged_decode_attention", &paged_decode_attention,
         "single-token GQA attention over the paged KV cache");
+  m.def("paged_decode_attention_fixed", &paged_decode_attention_fixed,
+        "decode attention whose order of sums never changes");
   m.def("paged_prefill_attention", &paged_prefill_attention,
         "varlen causal MFMA attention over the paged KV cache",
         pybind11::arg("out"), pybind11::arg("q"), pybind11::arg("k_cache"),
@@ -98,10 +98,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("topp_sample", &topp_sample, "temperature + top-p sampling per row");
   m.def("gather_kv_pages", &gather_kv_pages, "pages -> host-shaped buffer");
   m.def("stream_gemm", &stream_gemm,
-        "decode projection over packed rows and weights, M<=64");
+        "decode projection over packed rows and weights, M<=128");
   m.def("stream_gemm_experts", &stream_gemm_experts,
         "routed experts over packed rows and weights");
-  m.def("quant_packed", &quant_packed, "packed bf16 rows -> fp8 or e2m1");
   m.def("route_packed", &route_packed, "top-k router of packed rows");
   m.def("route_rows", &route_rows, "top-k router and expert order of rows");
   m.def("gather_pairs", &gather_pairs, "rows in expert order");

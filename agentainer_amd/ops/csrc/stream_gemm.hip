@@ -1,7 +1,6 @@
-// Decode projections (gfx950): x[M, K] @ W[N, K]^T for few rows, with bf16,
-// fp8 (e4m3, one scale per output) or mxfp4 (e2m1, one e8m0 scale per 32 k)
-// weights in the fragment-linear layouts of ops.pack_weight and
-// ops.quantize_weight_*, dense or as the experts of a mixture.
+// Decode projections (gfx950): x[M, K] @ W[N, K]^T for few rows, with bf16
+// weights in the fragment-linear layout of ops.pack_weight, dense or as the
+// experts of a mixture.
 //
 // HBM-bound: W is read once, everything else is small. Each workgroup owns NT
 // 16-column tiles and splits K over its WV waves, so no wave waits for another
@@ -26,9 +25,8 @@
 //
 // Up to 64 rows; 65 to 128 rows take wide_gemm_kernel below.
 //
-// bf16 and fp8: W is the A operand and x^T the B operand, so a lane ends up
-// with four consecutive output columns of one row. mxfp4: x is the A operand
-// and W with its scales the B operand, four rows of one column.
+// W is the A operand and x^T the B operand, so a lane ends up with four
+// consecutive output columns of one row.
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -41,36 +39,18 @@ namespace {
 typedef __bf16 bf16v8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16v4 __attribute__((ext_vector_type(4)));
 typedef int i32x4v __attribute__((ext_vector_type(4)));
-typedef int i32x8v __attribute__((ext_vector_type(8)));
 
 enum Mode { BF16 = 0, PARTS = 1, SILU = 2 };
-enum Weight { W_BF16 = 0, W_FP8 = 1, W_MXFP4 = 2 };
 constexpr int MAX_EXPERTS = 16;
 constexpr int MAX_PAIRS = 128;
 
-// k per fragment and bytes a lane holds of one
-template <int WT>
-struct Frag;
-template <>
-struct Frag<W_BF16> {
-  typedef bf16v8 type;
-  static constexpr int K = 32, BYTES = 16;
-};
-template <>
-struct Frag<W_FP8> {
-  typedef long type;
-  static constexpr int K = 32, BYTES = 8;
-};
-template <>
-struct Frag<W_MXFP4> {
-  typedef i32x4v type;
-  static constexpr int K = 128, BYTES = 16;
-};
+constexpr int FRAG_K = 32;           // k per fragment
+constexpr int LANE_BYTES = 16;       // what a lane holds of one
+constexpr int FRAG_BYTES = LANE_BYTES * WAVE;
 
 struct StreamArgs {
   void* out;
-  const char* x;        // packed rows of the weight's kind
-  const float* x_scale; // [rows of x] (fp8, mxfp4)
+  const char* x;        // packed rows
   int M, N, steps, steps_per_split;
   int x_groups;         // 16-row groups of the packed x
   // GROUPED
@@ -79,23 +59,20 @@ struct StreamArgs {
   int n_pairs, top_k, out_groups;
 };
 
-// weights and their scales (fp8: float [N]; mxfp4: e8m0 bytes) per expert
-template <int E>
-struct StreamWeights {
-  const char* w[E];
-  const void* scale[E];
-};
+// weights per expert
 template <bool GROUPED>
-using Weights = StreamWeights<GROUPED ? MAX_EXPERTS : 1>;
+struct Weights {
+  const char* w[GROUPED ? MAX_EXPERTS : 1];
+};
 
 // At most four waves a SIMD: aiming higher, the compiler moves the loads down
 // to their uses to save registers (gate_up at one row 40.9 instead of 40.2 us).
-template <int WT, int MODE, int MS, int NT, int WV, int U, bool GROUPED>
+template <int MODE, int MS, int NT, int WV, int U, bool GROUPED>
 __global__ __launch_bounds__(WV * WAVE)
 __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
     const StreamArgs a, const Weights<GROUPED> weights) {
-  typedef typename Frag<WT>::type frag;
-  constexpr int LB = Frag<WT>::BYTES, FB = LB * WAVE;
+  typedef bf16v8 frag;
+  constexpr int LB = LANE_BYTES, FB = FRAG_BYTES;
   const int lane = threadIdx.x % WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane % 16, lg = lane / 16;
@@ -139,16 +116,9 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
   const int x_groups = GROUPED ? a.x_groups : MS;
   const unsigned w_off = lane * LB;
   const char* wt[NT];
-  const unsigned char* sc[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
+  for (int nt = 0; nt < NT; ++nt)
     wt[nt] = weights.w[expert] + (long)tile_of(nt) * a.steps * FB;
-    sc[nt] = reinterpret_cast<const unsigned char*>(weights.scale[expert]) +
-             (long)tile_of(nt) * a.steps * WAVE;
-  }
-  // a scale operand has to be a VGPR, also the constant one
-  int unit_scale = 127;
-  if (WT == W_MXFP4) asm volatile("v_mov_b32 %0, 127" : "=v"(unit_scale));
 
   __shared__ f32x4 red[WV][MS][WAVE];
   constexpr int ITEMS = MS * WAVE;
@@ -175,9 +145,7 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
       for (int ms = 0; ms < MS; ++ms) acc[nt][ms] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     frag wa[U][NT], xa[U][MS], wb[U][NT], xb[U][MS];
-    int sa[U][NT], sb[U][NT];
-    auto load = [&](frag (&wf)[U][NT], frag (&xf)[U][MS], int (&sf)[U][NT],
-                    int step) {
+    auto load = [&](frag (&wf)[U][NT], frag (&xf)[U][MS], int step) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int s = min(step + u, last - 1);
@@ -186,7 +154,6 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
           const char* ws = wt[nt] + (long)s * FB;
           wf[u][nt] = __builtin_nontemporal_load(
               reinterpret_cast<const frag*>(ws + w_off));
-          if (WT == W_MXFP4) sf[u][nt] = (sc[nt] + (long)s * WAVE)[lane];
         }
         const char* xs = x + (long)s * (x_groups * FB);
 #pragma unroll
@@ -194,49 +161,36 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
           xf[u][ms] = *reinterpret_cast<const frag*>(xs + x_off[ms]);
       }
     };
-    auto multiply = [&](frag (&wf)[U][NT], frag (&xf)[U][MS], int (&sf)[U][NT],
-                        int step) {
+    auto multiply = [&](frag (&wf)[U][NT], frag (&xf)[U][MS], int step) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (u == 0 || step + u < last) {
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int ms = 0; ms < MS; ++ms) {
-              if constexpr (WT == W_BF16) {
-                acc[nt][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    wf[u][nt], xf[u][ms], acc[nt][ms], 0, 0, 0);
-              } else if constexpr (WT == W_FP8) {
-                acc[nt][ms] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-                    wf[u][nt], xf[u][ms], acc[nt][ms], 0, 0, 0);
-              } else {
-                const i32x4v xv = xf[u][ms], wv = wf[u][nt];
-                const i32x8v a8 = {xv[0], xv[1], xv[2], xv[3], 0, 0, 0, 0};
-                const i32x8v b8 = {wv[0], wv[1], wv[2], wv[3], 0, 0, 0, 0};
-                acc[nt][ms] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                    a8, b8, acc[nt][ms], 4, 4, 0, unit_scale, 0, sf[u][nt]);
-              }
-            }
+            for (int ms = 0; ms < MS; ++ms)
+              acc[nt][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  wf[u][nt], xf[u][ms], acc[nt][ms], 0, 0, 0);
         }
     };
     // No load of the main loop is conditional: behind a branch that may or may
     // not have issued loads the compiler has to wait for all of them.
     if (first < last) {
       int s = first;
-      load(wa, xa, sa, s);
+      load(wa, xa, s);
       while (s + 2 * U < last) {
-        load(wb, xb, sb, s + U);
-        multiply(wa, xa, sa, s);
-        load(wa, xa, sa, s + 2 * U);
-        multiply(wb, xb, sb, s + U);
+        load(wb, xb, s + U);
+        multiply(wa, xa, s);
+        load(wa, xa, s + 2 * U);
+        multiply(wb, xb, s + U);
         s += 2 * U;
       }
       if (s + U < last) {
-        load(wb, xb, sb, s + U);
-        multiply(wa, xa, sa, s);
-        multiply(wb, xb, sb, s + U);
+        load(wb, xb, s + U);
+        multiply(wa, xa, s);
+        multiply(wb, xb, s + U);
       } else {
-        multiply(wa, xa, sa, s);
+        multiply(wa, xa, s);
       }
     }
 
@@ -261,22 +215,8 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
 #pragma unroll
           for (int j = 0; j < 4; ++j) v[j] += o[j];
         }
-        // value j is slot m0 + j * dm, column n0 + j * dn of the tile
-        const int quad = (e % WAVE) / 16 * 4;
-        const int m0 = r0 + (e / WAVE) * 16 + (WT == W_MXFP4 ? quad : e % 16);
-        const int n0 = WT == W_MXFP4 ? e % 16 : quad;
-        constexpr int dm = WT == W_MXFP4 ? 1 : 0, dn = 1 - dm;
-        const int col = tile_of(nt) * 16 + n0;
-        if (WT != W_BF16) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int p = pair_of(min(m0 + j * dm, count - 1));
-            v[j] *= a.x_scale[GROUPED && MODE == SILU ? p / a.top_k : p];
-            if (WT == W_FP8)
-              v[j] *= reinterpret_cast<const float*>(
-                  weights.scale[expert])[col + j * dn];
-          }
-        }
+        // value j is slot m, column n + j
+        const int m = r0 + (e / WAVE) * 16 + e % 16;
         const int t = MODE == SILU ? (int)blockIdx.x * (NT / 2) + r / 2
                                    : (int)blockIdx.x * NT + nt;
         if (MODE == SILU && r % 2 == 0) {
@@ -291,7 +231,9 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
             v[j] = g / (1.f + __expf(-g)) * v[j];
           }
         }
-        auto at = [&](int m, int n) -> long {
+        const int n = t * 16 + (e % WAVE) / 16 * 4;
+        if (m >= count) continue;
+        auto at = [&]() -> long {
           if (MODE == SILU)
             return packed_at(pair_of(m), n, GROUPED ? a.out_groups : MS);
           if (MODE == PARTS && GROUPED) {
@@ -301,30 +243,16 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
           return (MODE == PARTS ? (long)blockIdx.y * a.M * a.N : 0) +
                  (long)m * a.N + n;
         };
-        const int n = t * 16 + n0;
-        if (dm == 0) {
-          if (m0 >= count) continue;
-          if (MODE == PARTS) {
-            const float f = GROUPED ? a.weight[pair_of(m0)] : 1.f;
+        if (MODE == PARTS) {
+          const float f = GROUPED ? a.weight[pair_of(m)] : 1.f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] *= f;
-            *reinterpret_cast<f32x4*>((float*)a.out + at(m0, n)) = v;
-          } else {
-            bf16x4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = f2bits(v[j]);
-            *reinterpret_cast<bf16x4*>((short*)a.out + at(m0, n)) = o;
-          }
+          for (int j = 0; j < 4; ++j) v[j] *= f;
+          *reinterpret_cast<f32x4*>((float*)a.out + at()) = v;
         } else {
+          bf16x4 o;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if (m0 + j >= count) continue;
-            if (MODE == PARTS)
-              ((float*)a.out)[at(m0 + j, n)] =
-                  v[j] * (GROUPED ? a.weight[pair_of(m0 + j)] : 1.f);
-            else
-              ((short*)a.out)[at(m0 + j, n)] = f2bits(v[j]);
-          }
+          for (int j = 0; j < 4; ++j) o[j] = f2bits(v[j]);
+          *reinterpret_cast<bf16x4*>((short*)a.out + at()) = o;
         }
       }
     }
@@ -332,23 +260,21 @@ __attribute__((amdgpu_waves_per_eu(WV / 4, 4))) void stream_gemm_kernel(
   }
 }
 
-template <int WT, int MODE, int MS, int NT, int WV, bool GROUPED>
+template <int MODE, int MS, int NT, int WV, bool GROUPED>
 void launch(const StreamArgs& a, const Weights<GROUPED>& w, int grid_y) {
   // fragments in flight: about 8 KB of W a wave, less where x takes the room
-  constexpr int U16 = NT * MS >= 8 ? 2 : NT * MS >= 2 ? 4 : 8;
-  constexpr int U = WT == W_FP8 ? 2 * U16
-                    : WT == W_MXFP4 ? (NT * MS >= 8 ? 2 : 4) : U16;
-  hipLaunchKernelGGL((stream_gemm_kernel<WT, MODE, MS, NT, WV, U, GROUPED>),
+  constexpr int U = NT * MS >= 8 ? 2 : NT * MS >= 2 ? 4 : 8;
+  hipLaunchKernelGGL((stream_gemm_kernel<MODE, MS, NT, WV, U, GROUPED>),
                      dim3((a.N / 16 + NT - 1) / NT, grid_y), dim3(WV * WAVE),
                      0, at::hip::getCurrentHIPStream(), a, w);
 }
 
-template <int WT, int MODE, int NT, int WV>
+template <int MODE, int NT, int WV>
 void by_rows(const StreamArgs& a, const Weights<false>& w, int split) {
   switch (packed_groups(a.M)) {
-    case 1: return launch<WT, MODE, 1, NT, WV, false>(a, w, split);
-    case 2: return launch<WT, MODE, 2, NT, WV, false>(a, w, split);
-    default: return launch<WT, MODE, 4, NT, WV, false>(a, w, split);
+    case 1: return launch<MODE, 1, NT, WV, false>(a, w, split);
+    case 2: return launch<MODE, 2, NT, WV, false>(a, w, split);
+    default: return launch<MODE, 4, NT, WV, false>(a, w, split);
   }
 }
 
@@ -363,30 +289,28 @@ void by_rows(const StreamArgs& a, const Weights<false>& w, int split) {
 //                           64: 213 (211)
 // More rows mean more x per byte of W: four tiles share a fragment then, where
 // N still gives enough workgroups.
-template <int WT>
 void dispatch(const StreamArgs& a, const Weights<false>& w, int mode,
               int split) {
-  if (mode == PARTS) return by_rows<WT, PARTS, 2, 8>(a, w, split);
+  if (mode == PARTS) return by_rows<PARTS, 2, 8>(a, w, split);
   if (mode == SILU)
-    return a.M <= 16 ? by_rows<WT, SILU, 2, 8>(a, w, 1)
-                     : by_rows<WT, SILU, 4, 4>(a, w, 1);
+    return a.M <= 16 ? by_rows<SILU, 2, 8>(a, w, 1)
+                     : by_rows<SILU, 4, 4>(a, w, 1);
   if (a.M > 16 && a.N >= 32768)
-    by_rows<WT, BF16, 4, 4>(a, w, 1);
+    by_rows<BF16, 4, 4>(a, w, 1);
   else
-    by_rows<WT, BF16, 2, 8>(a, w, 1);
+    by_rows<BF16, 2, 8>(a, w, 1);
 }
 
-template <int WT>
 void dispatch_grouped(const StreamArgs& a, const Weights<true>& w, int mode,
                       int experts) {
   // rows of one expert: a choice in 16 of a batch's fits one group up to 16
   // rows; larger batches take two groups at a time and come back for more
   if (mode == PARTS) {
-    if (a.n_pairs <= 16) launch<WT, PARTS, 1, 2, 8, true>(a, w, experts);
-    else launch<WT, PARTS, 2, 2, 8, true>(a, w, experts);
+    if (a.n_pairs <= 16) launch<PARTS, 1, 2, 8, true>(a, w, experts);
+    else launch<PARTS, 2, 2, 8, true>(a, w, experts);
   } else {
-    if (a.n_pairs <= 16) launch<WT, SILU, 1, 2, 8, true>(a, w, experts);
-    else launch<WT, SILU, 2, 2, 8, true>(a, w, experts);
+    if (a.n_pairs <= 16) launch<SILU, 1, 2, 8, true>(a, w, experts);
+    else launch<SILU, 2, 2, 8, true>(a, w, experts);
   }
 }
 
@@ -538,24 +462,13 @@ void launch_wide(const StreamArgs& a, const Weights<false>& w, int split) {
                      a.out, a.x, w.w[0], a.M, a.N, a.steps, a.steps_per_split);
 }
 
-int frag_k(long kind) { return kind == W_MXFP4 ? 128 : 32; }
-// bytes of a packed row group per k
-long x_bytes(long kind, long groups, long K) {
-  return groups * 16 * K * (kind == W_BF16 ? 4 : kind == W_FP8 ? 2 : 1) / 2;
+void check_weight(const torch::Tensor& w, long N, long K) {
+  TORCH_CHECK(w.is_contiguous() && w.scalar_type() == at::kBFloat16 &&
+              w.numel() == N * K);
 }
-
-void check_weight(const torch::Tensor& w, const torch::Tensor& ws, long kind,
-                  long N, long K) {
-  TORCH_CHECK(w.is_contiguous() && ws.is_contiguous());
-  if (kind == W_BF16) {
-    TORCH_CHECK(w.scalar_type() == at::kBFloat16 && w.numel() == N * K);
-  } else if (kind == W_FP8) {
-    TORCH_CHECK(w.scalar_type() == at::kByte && w.numel() == N * K &&
-                ws.scalar_type() == at::kFloat && ws.numel() == N);
-  } else {
-    TORCH_CHECK(w.scalar_type() == at::kByte && w.numel() == N * K / 2 &&
-                ws.scalar_type() == at::kByte && ws.numel() == N * K / 32);
-  }
+void check_packed(const torch::Tensor& x, long groups, long K) {
+  TORCH_CHECK(x.is_contiguous() && x.scalar_type() == at::kBFloat16 &&
+              x.numel() == groups * 16 * K);
 }
 
 }  // namespace
@@ -575,24 +488,16 @@ long stream_splits(long M, long N, long K) {
 }
 
 // mode 0: out bf16 [M, N]; 1: out fp32 [split, M, N]; 2: w = [gate; up], out
-// packed rows of N / 2. x: packed rows of K in the weight's kind (0 bf16,
-// 1 fp8 with x_scale, 2 mxfp4 with x_scale).
-void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor x_scale,
-                 torch::Tensor w, torch::Tensor w_scale, long kind, long M,
+// packed rows of N / 2. x: packed rows of K.
+void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w, long M,
                  long N, long K, long mode, long split) {
-  TORCH_CHECK(kind >= W_BF16 && kind <= W_MXFP4);
-  TORCH_CHECK(M >= 0 && M <= (kind == W_BF16 ? PACKED_ROWS : 64) &&
-                  N % 32 == 0 && K % frag_k(kind) == 0,
-              "stream_gemm: M <= 64 (bf16 128), N and K multiples of a "
-              "fragment");
+  TORCH_CHECK(M >= 0 && M <= PACKED_ROWS && N % 32 == 0 && K % FRAG_K == 0,
+              "stream_gemm: M <= 128, N and K multiples of a fragment");
   const long groups = packed_groups(M);
-  TORCH_CHECK(x.is_contiguous() &&
-              x.numel() * x.element_size() == x_bytes(kind, groups, K));
-  TORCH_CHECK(kind == W_BF16 || (x_scale.scalar_type() == at::kFloat &&
-                                 x_scale.numel() >= M));
-  check_weight(w, w_scale, kind, N, K);
+  check_packed(x, groups, K);
+  check_weight(w, N, K);
   TORCH_CHECK(out.is_contiguous());
-  const int steps = K / frag_k(kind);
+  const int steps = K / FRAG_K;
   TORCH_CHECK(split >= 1 && split <= steps &&
               (split - 1) * ((steps + split - 1) / split) < steps);
   TORCH_CHECK(mode >= BF16 && mode <= SILU);
@@ -608,8 +513,7 @@ void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor x_scale,
   StreamArgs a{};
   a.out = out.data_ptr();
   a.x = (const char*)x.data_ptr();
-  a.x_scale = kind == W_BF16 ? nullptr : x_scale.data_ptr<float>();
-  const Weights<false> wt{{(const char*)w.data_ptr()}, {w_scale.data_ptr()}};
+  const Weights<false> wt{{(const char*)w.data_ptr()}};
   a.M = M;
   a.N = N;
   a.steps = steps;
@@ -621,37 +525,28 @@ void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor x_scale,
     else launch_wide<BF16>(a, wt, 1);
     return;
   }
-  if (kind == W_BF16) dispatch<W_BF16>(a, wt, mode, split);
-  else if (kind == W_FP8) dispatch<W_FP8>(a, wt, mode, split);
-  else dispatch<W_MXFP4>(a, wt, mode, split);
+  dispatch(a, wt, mode, split);
 }
 
 // The experts' half of a mixture: mode 2 (SILU) turns packed rows of T tokens
 // into packed rows of T * top_k pairs, mode 1 (PARTS) those into fp32
 // [top_k, T, N], each times its pair's weight.
 void stream_gemm_experts(torch::Tensor out, torch::Tensor x,
-                         torch::Tensor x_scale, std::vector<torch::Tensor> w,
-                         std::vector<torch::Tensor> w_scale, long kind,
-                         torch::Tensor choice, torch::Tensor weight, long N,
-                         long K, long mode) {
+                         std::vector<torch::Tensor> w, torch::Tensor choice,
+                         torch::Tensor weight, long N, long K, long mode) {
   const int T = choice.size(0), top_k = choice.size(1);
   const int experts = w.size();
-  TORCH_CHECK(kind >= W_BF16 && kind <= W_MXFP4);
   TORCH_CHECK(choice.is_contiguous() && choice.scalar_type() == at::kInt &&
               weight.is_contiguous() && weight.scalar_type() == at::kFloat &&
               weight.numel() == choice.numel());
-  TORCH_CHECK(experts >= 1 && experts <= MAX_EXPERTS &&
-              w_scale.size() == w.size());
+  TORCH_CHECK(experts >= 1 && experts <= MAX_EXPERTS);
   TORCH_CHECK(T <= 64 && T * top_k <= MAX_PAIRS);
   TORCH_CHECK(mode == PARTS || mode == SILU);
-  TORCH_CHECK(N % 64 == 0 && K % frag_k(kind) == 0);
+  TORCH_CHECK(N % 64 == 0 && K % FRAG_K == 0);
   const int rows = mode == SILU ? T : T * top_k;
   const int x_groups = mode == SILU ? packed_groups(T) : (rows + 15) / 16;
   const int pair_groups = (T * top_k + 15) / 16;
-  TORCH_CHECK(x.is_contiguous() &&
-              x.numel() * x.element_size() == x_bytes(kind, x_groups, K));
-  TORCH_CHECK(kind == W_BF16 || (x_scale.scalar_type() == at::kFloat &&
-                                 x_scale.numel() >= rows));
+  check_packed(x, x_groups, K);
   TORCH_CHECK(out.is_contiguous() &&
               out.scalar_type() ==
                   (mode == PARTS ? at::kFloat : at::kBFloat16) &&
@@ -661,25 +556,21 @@ void stream_gemm_experts(torch::Tensor out, torch::Tensor x,
   StreamArgs a{};
   a.out = out.data_ptr();
   a.x = (const char*)x.data_ptr();
-  a.x_scale = kind == W_BF16 ? nullptr : x_scale.data_ptr<float>();
   Weights<true> wt{};
   for (int e = 0; e < experts; ++e) {
-    check_weight(w[e], w_scale[e], kind, N, K);
+    check_weight(w[e], N, K);
     wt.w[e] = (const char*)w[e].data_ptr();
-    wt.scale[e] = w_scale[e].data_ptr();
   }
   a.M = T;
   a.N = N;
-  a.steps = a.steps_per_split = K / frag_k(kind);
+  a.steps = a.steps_per_split = K / FRAG_K;
   a.x_groups = x_groups;
   a.choice = choice.data_ptr<int>();
   a.weight = weight.data_ptr<float>();
   a.n_pairs = T * top_k;
   a.top_k = top_k;
   a.out_groups = pair_groups;
-  if (kind == W_BF16) dispatch_grouped<W_BF16>(a, wt, mode, experts);
-  else if (kind == W_FP8) dispatch_grouped<W_FP8>(a, wt, mode, experts);
-  else dispatch_grouped<W_MXFP4>(a, wt, mode, experts);
+  dispatch_grouped(a, wt, mode, experts);
 }
 
 // ---------------------------------------------------------------------------
@@ -687,51 +578,17 @@ void stream_gemm_experts(torch::Tensor out, torch::Tensor x,
 
 namespace {
 
-// Eight values of a packed row as fp8 or e2m1 codes, in the packed order of
-// the kind.
-template <int WT>
-__device__ __forceinline__ void put_codes(unsigned char* xq, const bf16x8 v,
-                                          float inv, int row, int k,
-                                          int groups) {
-  if (WT == W_FP8) {
-    unsigned char o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f2fp8(bits2f(v[j]) * inv);
-    *reinterpret_cast<uint2*>(xq + packed_at(row, k, groups)) =
-        *reinterpret_cast<uint2*>(o);
-  } else {
-    unsigned char o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] = f2e2m1(bits2f(v[2 * j]) * inv) |
-             (f2e2m1(bits2f(v[2 * j + 1]) * inv) << 4);
-    // 128 k a fragment, 32 consecutive k (16 bytes) a lane
-    const long at = ((long)(k / 128) * groups + row / 16) * 1024 +
-                    ((k % 128) / 32 * 16 + row % 16) * 16 + (k % 32) / 2;
-    *reinterpret_cast<unsigned int*>(xq + at) =
-        *reinterpret_cast<unsigned int*>(o);
-  }
-}
-
-// largest code of a kind
-template <int WT>
-constexpr float code_max() {
-  return WT == W_FP8 ? 448.f : 6.f;
-}
-
 // residual += sum of the parts (rounded once), out = rmsnorm(residual) as
-// packed rows (ms > 0) or row-major (ms = 0); WT fp8 or mxfp4: as codes with
-// the row's scale. One row per workgroup, held in registers between the
-// reductions and the stores. n_parts 0: only the norm.
-template <int VPT, int WT>
+// packed rows (ms > 0) or row-major (ms = 0). One row per workgroup, held in
+// registers between the reduction and the stores. n_parts 0: only the norm.
+template <int VPT>
 __global__ __launch_bounds__(512) void add_parts_rmsnorm_kernel(
-    void* __restrict__ out, float* __restrict__ out_scale,
-    short* __restrict__ residual, const float* __restrict__ parts, int n_parts,
+    short* __restrict__ out, short* __restrict__ residual, const float* __restrict__ parts, int n_parts,
     long part_stride, const short* __restrict__ w, float eps, int H, int ms) {
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
   const long base = (long)row * H;
-  __shared__ float red[2][8];
+  __shared__ float red[8];
   bf16x8 v[VPT];
   float ss = 0.f;
 #pragma unroll
@@ -764,42 +621,22 @@ __global__ __launch_bounds__(512) void add_parts_rmsnorm_kernel(
     }
   }
   ss = wave_sum(ss);
-  if ((tid & (WAVE - 1)) == 0) red[0][tid / WAVE] = ss;
+  if ((tid & (WAVE - 1)) == 0) red[tid / WAVE] = ss;
   __syncthreads();
   ss = 0.f;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) ss += red[0][q];
+  for (int q = 0; q < 8; ++q) ss += red[q];
   const float rms = rsqrtf(ss / (float)H + eps);
-  float mx = 0.f;
 #pragma unroll
   for (int r = 0; r < VPT; ++r) {
     const int i = (tid + r * 512) * 8;
     if (i >= H) continue;
     const bf16x8 wv = *reinterpret_cast<const bf16x8*>(w + i);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 8; ++j)
       v[r][j] = f2bits(bits2f(v[r][j]) * rms * bits2f(wv[j]));
-      mx = fmaxf(mx, fabsf(bits2f(v[r][j])));
-    }
-    if (WT == W_BF16)
-      *reinterpret_cast<bf16x8*>(
-          (short*)out + (ms ? packed_at(row, i, ms) : base + i)) = v[r];
-  }
-  if constexpr (WT != W_BF16) {
-    mx = wave_max(mx);
-    if ((tid & (WAVE - 1)) == 0) red[1][tid / WAVE] = mx;
-    __syncthreads();
-    mx = 0.f;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) mx = fmaxf(mx, red[1][q]);
-    const float s = fmaxf(mx, 1e-8f) / code_max<WT>();
-    const float inv = 1.0f / s;
-    if (tid == 0) out_scale[row] = s;
-#pragma unroll
-    for (int r = 0; r < VPT; ++r) {
-      const int i = (tid + r * 512) * 8;
-      if (i < H) put_codes<WT>((unsigned char*)out, v[r], inv, row, i, ms);
-    }
+    *reinterpret_cast<bf16x8*>(out + (ms ? packed_at(row, i, ms) : base + i)) =
+        v[r];
   }
 }
 
@@ -815,27 +652,20 @@ __global__ void pack_rows_kernel(short* __restrict__ out,
 
 }  // namespace
 
-// kind 0: out bf16, packed or row-major; 1, 2: out codes of packed rows and
-// their scales
-void add_parts_rmsnorm(torch::Tensor out, torch::Tensor out_scale,
-                       torch::Tensor residual,
+// out: packed or row-major rows
+void add_parts_rmsnorm(torch::Tensor out, torch::Tensor residual,
                        c10::optional<torch::Tensor> parts, torch::Tensor w,
-                       double eps, bool packed, long kind) {
+                       double eps, bool packed) {
   TORCH_CHECK(residual.is_contiguous() && w.is_contiguous() &&
               out.is_contiguous());
   TORCH_CHECK(residual.scalar_type() == at::kBFloat16 &&
-              w.scalar_type() == at::kBFloat16);
+              w.scalar_type() == at::kBFloat16 &&
+              out.scalar_type() == at::kBFloat16);
   const int T = residual.size(0), H = residual.size(1);
-  TORCH_CHECK(kind >= W_BF16 && kind <= W_MXFP4 && (packed || kind == W_BF16));
   TORCH_CHECK(w.numel() == H && H % 8 == 0 && H <= 16384);
-  TORCH_CHECK(!packed || (T <= PACKED_ROWS && H % frag_k(kind) == 0));
+  TORCH_CHECK(!packed || (T <= PACKED_ROWS && H % FRAG_K == 0));
   const int ms = packed ? packed_groups(T) : 0;
-  TORCH_CHECK(out.scalar_type() ==
-              (kind == W_BF16 ? at::kBFloat16 : at::kByte));
-  TORCH_CHECK(out.numel() * out.element_size() ==
-              (packed ? x_bytes(kind, ms, H) : (long)T * H * 2));
-  TORCH_CHECK(kind == W_BF16 || (out_scale.scalar_type() == at::kFloat &&
-                                 out_scale.numel() >= T));
+  TORCH_CHECK(out.numel() == (packed ? (long)ms * 16 : (long)T) * H);
   int n_parts = 0;
   const float* pp = nullptr;
   if (parts.has_value()) {
@@ -847,22 +677,14 @@ void add_parts_rmsnorm(torch::Tensor out, torch::Tensor out_scale,
   }
   if (T == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-#define AP_LAUNCH(VPT, WT)                                                     \
-  hipLaunchKernelGGL((add_parts_rmsnorm_kernel<VPT, WT>), dim3(T), dim3(512),  \
-                     0, stream, out.data_ptr(),                                \
-                     WT == W_BF16 ? nullptr : out_scale.data_ptr<float>(),     \
+#define AP_LAUNCH(VPT)                                                         \
+  hipLaunchKernelGGL((add_parts_rmsnorm_kernel<VPT>), dim3(T), dim3(512), 0,   \
+                     stream, (short*)out.data_ptr(),                           \
                      (short*)residual.data_ptr(), pp, n_parts, (long)T * H,    \
                      (const short*)w.data_ptr(), (float)eps, H, ms)
-#define AP_KIND(VPT)                                                           \
-  do {                                                                         \
-    if (kind == W_BF16) AP_LAUNCH(VPT, W_BF16);                                \
-    else if (kind == W_FP8) AP_LAUNCH(VPT, W_FP8);                             \
-    else AP_LAUNCH(VPT, W_MXFP4);                                              \
-  } while (0)
-  if (H <= 4096) AP_KIND(1);
-  else if (H <= 8192) AP_KIND(2);
-  else AP_KIND(4);
-#undef AP_KIND
+  if (H <= 4096) AP_LAUNCH(1);
+  else if (H <= 8192) AP_LAUNCH(2);
+  else AP_LAUNCH(4);
 #undef AP_LAUNCH
 }
 
@@ -882,37 +704,9 @@ void pack_rows(torch::Tensor out, torch::Tensor x) {
 }
 
 // ---------------------------------------------------------------------------
-// Packed bf16 rows quantized for fp8 or mxfp4 weights, and the router.
+// The router.
 
 namespace {
-
-// One row per workgroup: largest magnitude, then the codes in the packed
-// order of the kind (fp8: scale to 448, e2m1: to 6).
-template <int WT>
-__global__ __launch_bounds__(256) void quant_packed_kernel(
-    unsigned char* __restrict__ xq, float* __restrict__ scale,
-    const short* __restrict__ x, int K, int groups) {
-  const int row = blockIdx.x;
-  __shared__ float red[4];
-  float mx = 0.f;
-  for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
-    const bf16x8 v =
-        *reinterpret_cast<const bf16x8*>(x + packed_at(row, k, groups));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(bits2f(v[j])));
-  }
-  mx = wave_max(mx);
-  if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const float s = fmaxf(mx, 1e-8f) / code_max<WT>();
-  const float inv = 1.0f / s;
-  if (threadIdx.x == 0) scale[row] = s;
-  for (int k = threadIdx.x * 8; k < K; k += 256 * 8)
-    put_codes<WT>(
-        xq, *reinterpret_cast<const bf16x8*>(x + packed_at(row, k, groups)),
-        inv, row, k, groups);
-}
 
 // Router of one token per workgroup: fp32 logits of E experts, softmax, the
 // top_k largest (lowest index first among equals), weights that sum to 1.
@@ -968,30 +762,6 @@ __global__ __launch_bounds__(256) void route_packed_kernel(
 }
 
 }  // namespace
-
-// groups: 16-row groups of the packed x; rows 0 .. rows-1 are quantized
-void quant_packed(torch::Tensor xq, torch::Tensor scale, torch::Tensor x,
-                  long kind, long rows, long K) {
-  TORCH_CHECK(kind == W_FP8 || kind == W_MXFP4);
-  TORCH_CHECK(x.is_contiguous() && x.scalar_type() == at::kBFloat16 &&
-              K % frag_k(kind) == 0 && x.numel() % (16 * K) == 0);
-  const int groups = x.numel() / (16 * K);
-  TORCH_CHECK(rows <= groups * 16 && scale.numel() >= rows &&
-              scale.scalar_type() == at::kFloat);
-  TORCH_CHECK(xq.is_contiguous() && xq.scalar_type() == at::kByte &&
-              xq.numel() == x_bytes(kind, groups, K));
-  if (rows == 0) return;
-  auto stream = at::hip::getCurrentHIPStream();
-  if (kind == W_FP8)
-    hipLaunchKernelGGL((quant_packed_kernel<W_FP8>), dim3(rows), dim3(256), 0,
-                       stream, xq.data_ptr<uint8_t>(), scale.data_ptr<float>(),
-                       (const short*)x.data_ptr(), (int)K, groups);
-  else
-    hipLaunchKernelGGL((quant_packed_kernel<W_MXFP4>), dim3(rows), dim3(256),
-                       0, stream, xq.data_ptr<uint8_t>(),
-                       scale.data_ptr<float>(), (const short*)x.data_ptr(),
-                       (int)K, groups);
-}
 
 void route_packed(torch::Tensor choice, torch::Tensor weight, torch::Tensor x,
                   torch::Tensor router) {

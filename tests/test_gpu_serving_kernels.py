@@ -255,51 +255,13 @@ def test_packed_attention_outputs_are_the_rows():
             assert torch.equal(pk[slot], rows.view(-1))
 
 
-@pytest.mark.parametrize("kind", ["fp8", "mxfp4"])
-@pytest.mark.parametrize("T,N,K", [(1, 64, 256), (17, 192, 512),
-                                   (64, 4096, 4096), (33, 32832, 256)])
-def test_stream_quantized_projections(kind, T, N, K):
-    """Against the row-major quantized products of the same codes: the same
-    values, summed in another order."""
-    gen = torch.Generator(device=DEV).manual_seed(T + N)
-    x = torch.randn(T, K, generator=gen, device=DEV).to(torch.bfloat16)
-    w = torch.randn(N, K, generator=gen, device=DEV).to(torch.bfloat16)
-    quant = (ops.quantize_weight_fp8 if kind == "fp8"
-             else ops.quantize_weight_mxfp4)
-    qt = (kind, *quant(w), N)
-    want = ops.linear_quant(x, qt)
-    xp = ops.pack_rows(x)
-    got = ops.stream_linear(xp, T, qt, N, K)
-    # two bf16 roundings of sums that differ in their last fp32 bits
-    assert bool(((got.float() - want.float()).abs()
-                 <= 2.0 ** -7 * want.float().abs() + 1e-3).all())
-    parts = ops.stream_parts(xp, T, qt, N, K)
-    assert _rel(parts.sum(0), want) < 2.0 ** -8
-    act = ops.stream_gate_up(xp, T, qt, N, K)
-    g, u = parts.sum(0).chunk(2, dim=1)
-    exp = torch.nn.functional.silu(g) * u
-    rows = act[_row_slots(T, N // 2)].view(T, N // 2)
-    assert _rel(rows, exp) < 2.0 ** -8
-    # codes written by the norm are those of its bf16 rows, quantized
-    if K % 128 == 0:
-        ln = torch.rand(K, generator=gen, device=DEV).to(torch.bfloat16)
-        bf = ops.add_parts_rmsnorm(x.clone(), parts[:, :, :K].contiguous()
-                                   if N >= K else None, ln, 1e-5)
-        codes = ops.add_parts_rmsnorm(x.clone(), parts[:, :, :K].contiguous()
-                                      if N >= K else None, ln, 1e-5,
-                                      for_weight=qt)
-        assert torch.equal(ops.stream_linear(codes, T, qt, N, K),
-                           ops.stream_linear(bf, T, qt, N, K))
-
-
-@pytest.mark.parametrize("kind", ["bf16", "fp8", "mxfp4"])
 @pytest.mark.parametrize("T,E,top_k,spread", [
     (1, 8, 2, 1.0), (3, 4, 2, 1.0), (16, 8, 2, 1.0), (32, 8, 2, 1.0),
     (64, 8, 2, 1.0), (7, 16, 8, 1.0), (128 // 3, 5, 3, 1.0),
     (64, 8, 2, 0.0),   # every token chooses the same experts: many row groups
     (9, 1, 1, 1.0),
 ])
-def test_stream_experts(kind, T, E, top_k, spread):
+def test_stream_experts(T, E, top_k, spread):
     """Routing and both expert projections against the plain computation."""
     H, inter = 256, 512
     gen = torch.Generator(device=DEV).manual_seed(T * E)
@@ -318,33 +280,19 @@ def test_stream_experts(kind, T, E, top_k, spread):
     want_w = (top / top.sum(-1, keepdim=True)).float()
     # logits of about 16 summed in fp32
     assert bool(((weight - want_w).abs() <= 1e-4).all())
-    if kind == "bf16":
-        gu_w = [ops.pack_weight(w) for w in gus]
-        dn_w = [ops.pack_weight(w) for w in dns]
-    else:
-        quant = (ops.quantize_weight_fp8 if kind == "fp8"
-                 else ops.quantize_weight_mxfp4)
-        gu_w = [(kind, *quant(w), 2 * inter) for w in gus]
-        dn_w = [(kind, *quant(w), H) for w in dns]
+    gu_w = [ops.pack_weight(w) for w in gus]
+    dn_w = [ops.pack_weight(w) for w in dns]
     parts = ops.stream_experts(xp, T, choice, weight, gu_w, dn_w, inter, H)
     assert parts.shape == (top_k, T, H)
     want = torch.zeros(T, H, device=DEV)
     for e in range(E):
         w_e = torch.where(who == e, weight, torch.zeros_like(weight)).sum(-1)
-        if kind == "bf16":
-            g, u = (x.float() @ gus[e].float().t()).chunk(2, dim=1)
-            act = (torch.nn.functional.silu(g) * u).to(torch.bfloat16)
-            y = act.float() @ dns[e].float().t()
-        else:  # the dense projections of the same codes
-            act = ops.stream_gate_up(xp, T, gu_w[e], 2 * inter, H)
-            y = ops.stream_parts(act, T, dn_w[e], H, inter).sum(0)
+        g, u = (x.float() @ gus[e].float().t()).chunk(2, dim=1)
+        act = (torch.nn.functional.silu(g) * u).to(torch.bfloat16)
+        y = act.float() @ dns[e].float().t()
         want += w_e[:, None] * y
-    # bf16: activations may round to the other neighbour (2^-8 of a value).
-    # Quantized: one activation in a thousand does, and of those one in 16
-    # (fp8, steps of 2^-3) or in a hundred (e2m1, steps of up to a half)
-    # changes its code
-    assert _rel(parts.sum(0), want) < {"bf16": 2.0 ** -8, "fp8": 2.0 ** -9,
-                                       "mxfp4": 2.0 ** -7}[kind]
+    # activations may round to the other neighbour (2^-8 of a value)
+    assert _rel(parts.sum(0), want) < 2.0 ** -8
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
@@ -461,3 +409,119 @@ def test_attention_rows_off_alignment():
     ops.paged_prefill_attention(out, q, *args, max_qlen=1)
     ops.paged_prefill_attention(want, q.contiguous(), *args, max_qlen=1)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n_q,n_kv,PS,lens,width", [
+    (32, 8, 16, [1, 63, 64, 65, 511, 512, 513, 900], 0),  # chunks and runs
+    (8, 8, 8, [70, 3], 0),
+    (16, 8, 24, [255, 2], 64),
+    (64, 8, 16, [300, 1], 0),
+])
+def test_fixed_decode_attention_edges(dtype, n_q, n_kv, PS, lens, width):
+    D, B = 128, len(lens)
+    kc, vc, table = _paged(lens, n_kv, D, PS, dtype, width, seed=n_q + PS)
+    gen = torch.Generator().manual_seed(7)
+    q = torch.randn(B, n_q, D, generator=gen).to(torch.bfloat16)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    scale = 1.0 / math.sqrt(D)
+    out = torch.zeros(B + 1, n_q, D, dtype=torch.bfloat16, device=DEV)
+    ops.paged_decode_attention_fixed(out[:B], q.to(DEV), kc.to(DEV),
+                                     vc.to(DEV), table.to(DEV), sl.to(DEV),
+                                     scale)
+    qr = q.float()
+    if dtype != torch.bfloat16:  # queries in e4m3, one scale per head
+        step = qr.abs().amax(-1, keepdim=True).clamp(min=1e-8) / 448.0
+        qr = (qr * (1.0 / step)).to(torch.float8_e4m3fn).float() * step
+    want = torch.zeros(B, n_q, D)
+    ref.paged_decode_attention(want, qr, kc.float(), vc.float(), table, sl,
+                               scale)
+    # the result's own rounding, and fp32 sums of a few hundred terms
+    err = (out[:B].float().cpu() - want).abs()
+    vmax = float(vc.float().nan_to_num().abs().max())
+    assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * vmax).all())
+    assert not out[B].any()
+
+
+def _decode_state(cfg, lens, kv_dtype, n_layers, seed, PS=16):
+    """Caches, metadata and tokens of a decode step over `lens` cached
+    tokens."""
+    from agentainer_amd.models.llama import AttnMetadata
+    caches = []
+    for i in range(n_layers):
+        kc, vc, table = _paged([n + 1 for n in lens], cfg.n_kv_heads,
+                               cfg.head_dim, PS, torch.bfloat16, seed=seed)
+        caches.append((kc.nan_to_num().to(kv_dtype).to(DEV),
+                       vc.nan_to_num().to(kv_dtype).to(DEV)))
+    pos = torch.tensor(lens, dtype=torch.int32)
+    slots = torch.stack([table[b, n // PS].long() * PS + n % PS
+                         for b, n in enumerate(lens)])
+    md = AttnMetadata(page_table=table.to(DEV), seq_lens=(pos + 1).to(DEV),
+                      slot_mapping=slots.to(DEV), positions=pos.to(DEV))
+    gen = torch.Generator().manual_seed(seed)
+    ids = torch.randint(0, cfg.vocab_size, (len(lens),), generator=gen)
+    return caches, md, ids.to(DEV)
+
+
+@pytest.mark.parametrize("name,quant", [
+    ("tiny-llama", "fp8"), ("tiny-llama", "mxfp4"),
+    ("tiny-mixtral", "fp8"), ("tiny-mixtral", "mxfp4")])
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("T", [1, 13, 64])
+@torch.no_grad()
+def test_quantized_decode_is_row_major(name, quant, kv_dtype, T):
+    """A decode step over quantized weights is, bit for bit, the row-major
+    chain of the single ops: its codes depend on every order of sums."""
+    from agentainer_amd.models.llama import LLAMA_CONFIGS, LlamaForCausalLM
+    from agentainer_amd.models.mixtral import (MIXTRAL_CONFIGS,
+                                               MixtralForCausalLM)
+    moe = name in MIXTRAL_CONFIGS
+    cfg = (MIXTRAL_CONFIGS if moe else LLAMA_CONFIGS)[name]
+    model = (MixtralForCausalLM if moe else LlamaForCausalLM)(cfg, DEV)
+    if moe:
+        model.pack_decode_weights(expert_fp8=quant == "fp8",
+                                  expert_fp4=quant == "mxfp4")
+    else:
+        model.pack_decode_weights(dense_quant=quant)
+    lens = [3 + 29 * i for i in range(T)]
+    caches, md, ids = _decode_state(cfg, lens, kv_dtype, cfg.n_layers, T)
+    copies = [(k.clone(), v.clone()) for k, v in caches]
+    got = model(ids, md, caches)
+
+    D, nq, nkv, eps = cfg.head_dim, cfg.n_heads, cfg.n_kv_heads, cfg.norm_eps
+    x = torch.nn.functional.embedding(ids, model.embed)
+    res = None
+    for layer, (kc, vc) in zip(model.layers, copies):
+        h = torch.empty_like(x)
+        if res is None:
+            res = x.clone()
+            ops.rmsnorm(h, x, layer.input_ln, eps)
+        else:
+            ops.fused_add_rmsnorm(h, x, res, layer.input_ln, eps)
+        at = layer.attn
+        qkv = (ops.linear(h, at.qkv_proj, at.qkv_packed) if moe
+               else ops.linear_quant(h, at.qkv_q))
+        q, k, v = qkv.split([nq * D, nkv * D, nkv * D], dim=1)
+        q = q.unflatten(1, (nq, D))
+        ops.rope_append(q, k.unflatten(1, (nkv, D)), v.unflatten(1, (nkv, D)),
+                        kc, vc, model.cos_sin, md.positions, md.slot_mapping)
+        o = torch.empty(T, nq, D, dtype=torch.bfloat16, device=DEV)
+        ops.paged_decode_attention_fixed(o, q, kc, vc, md.page_table,
+                                         md.seq_lens, at.scale)
+        o = o.view(T, nq * D)
+        x = (ops.linear(o, at.o_proj, at.o_packed) if moe
+             else ops.linear_quant(o, at.o_q))
+        h = torch.empty_like(x)
+        ops.fused_add_rmsnorm(h, x, res, layer.post_ln, eps)
+        if moe:
+            x = layer.moe(h)
+            continue
+        gu = ops.linear_quant(h, layer.mlp.gate_up_q)
+        inter = layer.mlp.inter
+        act = torch.empty(T, inter, dtype=torch.bfloat16, device=DEV)
+        ops.silu_mul(act, gu[:, :inter], gu[:, inter:])
+        x = ops.linear_quant(act, layer.mlp.down_q)
+    h = torch.empty_like(x)
+    ops.fused_add_rmsnorm(h, x, res, model.final_ln, eps)
+    want = ops.linear(h, model.lm_head, model.lm_head_packed)
+    assert torch.equal(got, want)
