@@ -108,10 +108,44 @@ def test_decode_attention_edges(dtype, n_q, n_kv, PS, lens, width):
     want = torch.zeros(B, n_q, D)
     ref.paged_decode_attention(want, q.float(), kc.float(), vc.float(), table,
                                sl, scale)
-    # probabilities keep 16 bits; the rest is the result's own rounding
+    # the result's own rounding, and fp32 sums of up to 8190 terms
     err = (out.float().cpu() - want).abs()
     vmax = float(vc.float().nan_to_num().abs().max())
     assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * vmax).all())
+
+
+@pytest.mark.parametrize("n_q,n_kv", [(8, 8), (32, 8), (64, 8)])
+def test_decode_probabilities_keep_32_bits(n_q, n_kv):
+    """Two tokens with nearly the same score and opposite values beside one
+    without any: the result is the difference of two probabilities near 1/3,
+    and shows every bit that one of them lost on its way through the
+    product."""
+    D, PS, B = 128, 16, 64
+    gen = torch.Generator().manual_seed(n_q)
+    q = torch.randn(B, n_q, D, generator=gen).to(torch.bfloat16)
+    kc = torch.zeros(B, n_kv, D // 8, PS, 8, dtype=torch.bfloat16)
+    kc[:, :, :, :2] = (torch.randn(B, n_kv, D // 8, 1, 8, generator=gen)
+                       + 2e-3 * torch.randn(B, n_kv, D // 8, 2, 8,
+                                            generator=gen))
+    vc = torch.zeros(B, n_kv, PS, D, dtype=torch.bfloat16)
+    vc[:, :, 0], vc[:, :, 1] = 1.0, -1.0
+    table = torch.arange(B, dtype=torch.int32)[:, None]
+    sl = torch.full((B,), 3, dtype=torch.int32)
+    scale = 0.002
+    out = torch.zeros(B, n_q, D, dtype=torch.bfloat16, device=DEV)
+    ops.paged_decode_attention(out, q.to(DEV), kc.to(DEV), vc.to(DEV),
+                               table.to(DEV), sl.to(DEV), scale)
+    keys = kc[:, :, :, :3].double().permute(0, 1, 3, 2, 4).reshape(
+        B, n_kv, 3, D).repeat_interleave(n_q // n_kv, dim=1)
+    s = (keys @ q.double()[..., None])[..., 0] * scale
+    p = torch.softmax(s, -1)
+    want = (p[..., 0] - p[..., 1])[..., None]
+    assert 1e-5 < want.abs().max() < 1e-3
+    # half a bf16 step of the result; two probabilities of 1/3, each off by a
+    # few 2^-24 of itself (its exponent, its exponential, the quotient). With
+    # 16 bits they are off by 2^-18 of themselves, 1.3e-6 each
+    assert bool(((out.double().cpu() - want).abs()
+                 <= 2.0 ** -8 * want.abs() + 2.0 ** -22).all())
 
 
 def test_rope_append_decode_is_both_steps():
