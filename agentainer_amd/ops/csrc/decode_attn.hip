@@ -183,7 +183,7 @@ __global__ __launch_bounds__(WAVES * WAVE, 3) void decode_attn_kernel(
   }
 
   // one tile: K chunk (token 16i + col, d8 = 4s + lg), V chunk (token
-  // 4i + lg, dims 8*col ..+8). Tokens past the run repeat its last one, so
+  // 4i + lg, dims 8*col ..+8). Tokens past the run load its last one, so
   // nothing stale is ever multiplied.
   raw rk[2][4], rv[8];
   // pages of a tile's two groups, looked up one tile ahead
@@ -253,6 +253,13 @@ __global__ __launch_bounds__(WAVES * WAVE, 3) void decode_attn_kernel(
     look(t + WAVES * TILE);
   }
   for (; t < t_end; t += WAVES * TILE) {
+    const int left = t_end - t;  // tokens of this tile that exist
+    if (left < TILE) {
+      // the others' probabilities are 0: their values have to be finite
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (4 * i + w_slot >= left) rv[i] = raw{};
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int row = 4 * i + w_slot;
@@ -271,7 +278,6 @@ __global__ __launch_bounds__(WAVES * WAVE, 3) void decode_attn_kernel(
             *reinterpret_cast<const bf16v8*>(&kv), qf[st], s[i], 0, 0, 0);
       }
     }
-    const int left = t_end - t;  // tokens of this tile that exist
     if (t + WAVES * TILE < t_end) {
       load(t + WAVES * TILE);
       look(t + 2 * WAVES * TILE);
@@ -349,7 +355,12 @@ __global__ __launch_bounds__(WAVES * WAVE, 3) void decode_attn_kernel(
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float v = o[dt][r] + other_half(o[dt][r]);
+        // A low part is often exactly 0, and 0 times an infinite value is
+        // NaN; the upper parts of a probability above 0 are above 0 too, so
+        // their half alone has the answer whenever it is not finite.
+        const float low = other_half(o[dt][r]);
+        const float v = __builtin_isfinite(o[dt][r]) ? o[dt][r] + low
+                                                     : o[dt][r];
         if (col < RATIO) mine[col * PART + dt * 16 + lg * 4 + r] = v;
       }
     if (lg == 0 && col < RATIO) {

@@ -148,6 +148,39 @@ def test_decode_probabilities_keep_32_bits(n_q, n_kv):
                  <= 2.0 ** -8 * want.abs() + 2.0 ** -22).all())
 
 
+@pytest.mark.parametrize("n_q,n_kv", [(8, 8), (8, 2), (16, 2)])
+def test_decode_infinite_values(n_q, n_kv):
+    """An infinite value of a token that is attended to makes the result
+    infinite, wherever in a tile, a run or a wave the token is; two of
+    opposite signs, or a NaN, make it NaN; the other columns stay."""
+    D, PS = 128, 16
+    lens = [1, 2, 31, 32, 33, 128, 129, 5000]
+    kc, vc, table = _paged(lens, n_kv, D, PS, torch.bfloat16, 512, seed=3)
+    inf = math.inf
+    for b, n in enumerate(lens):
+        for at, col, val in ((n - 1, 3, inf), (0, 70, -inf), (n // 2, 127, inf),
+                             (n - 1, 5, math.nan), (n - 1, 6, inf),
+                             (0, 6, -inf)):
+            vc[table[b, at // PS], :, at % PS, col] = val
+    gen = torch.Generator().manual_seed(8)
+    q = torch.randn(len(lens), n_q, D, generator=gen).to(torch.bfloat16)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    out = torch.zeros(len(lens), n_q, D, dtype=torch.bfloat16, device=DEV)
+    ops.paged_decode_attention(out, q.to(DEV), kc.to(DEV), vc.to(DEV),
+                               table.to(DEV), sl.to(DEV), 0.05)
+    want = torch.zeros(len(lens), n_q, D)
+    ref.paged_decode_attention(want, q.float(), kc.float(), vc.float(), table,
+                               sl, 0.05)
+    got = out.float().cpu()
+    assert want.isinf().any() and want.isnan().any()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    assert bool(((got - want).abs()[fine]
+                 <= 2.0 ** -8 * want.abs()[fine] + 2.0 ** -11).all())
+
+
 def test_rope_append_decode_is_both_steps():
     """Rotation, append and attention in one call against the single ops;
     a padded row (no tokens) is left alone, dirty counters do not matter."""
