@@ -184,8 +184,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
 
   // staging: per 16-token group i of a tile this thread moves K chunk
   // (token 16i + tid%16, d8 = tid/16) and V chunk (token 16i + tid/16,
-  // columns 8 * (tid%16)). Tokens past the last visible one repeat it, so
-  // nothing stale is ever multiplied.
+  // columns 8 * (tid%16)). Tokens past the last visible one load it again, so
+  // nothing stale is ever multiplied, and their values are zeroed on the way
+  // to LDS: under a probability of 0 an infinite one would make NaN.
   typedef typename Raw<CT>::type raw;
   raw st_k[4], st_v[4];
   const int lo = threadIdx.x % 16, hi = threadIdx.x / 16;
@@ -209,7 +210,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
       st_v[i] = *reinterpret_cast<const raw*>(v_cache + vb * D + lo * 8);
     }
   };
-  auto stage_write = [&](int buf) {
+  auto stage_write = [&](int buf, int t) {
+    const int left = kv_end - t * KVBLK;
+    if (left < KVBLK) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (16 * i + hi >= left) st_v[i] = raw{};
+    }
     short* kl = lds + buf * (K_TILE + V_TILE);
     short* vl = kl + K_TILE;
 #pragma unroll
@@ -223,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
 
   if (t0 < t1) {
     stage_load(t0);
-    stage_write(0);
+    stage_write(0, t0);
   }
   __syncthreads();
   // fragment bases: K chunk of (token l32, d8 = h); V block of the 16-lane
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
         }
       }
     }
-    if (has_next) stage_write(buf ^ 1);
+    if (has_next) stage_write(buf ^ 1, t + 1);
     __syncthreads();
     buf ^= 1;
   }

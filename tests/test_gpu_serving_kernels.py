@@ -181,6 +181,46 @@ def test_decode_infinite_values(n_q, n_kv):
                  <= 2.0 ** -8 * want.abs()[fine] + 2.0 ** -11).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("width", [0, 512])  # one run, and split runs
+def test_prefill_infinite_values(dtype, width):
+    """A row's own token, or one that every row sees, with values that are not
+    finite. (Rows that a tile masks from such a token get NaN of it.)"""
+    n_q, n_kv, D, PS = 8, 2, 128, 16
+    specs = [(0, 1), (30, 1), (31, 1), (62, 1), (63, 1), (700, 1), (2, 33)]
+    kc, vc, table = _paged([c + n for c, n in specs], n_kv, D, PS,
+                           torch.bfloat16, width, seed=4)
+    special = math.inf if dtype == torch.bfloat16 else math.nan  # e4m3: no inf
+    for b, (c, n) in enumerate(specs):
+        for at, col in ((c + n - 1, 3), (0, 127)):
+            vc[table[b, at // PS], :, at % PS, col] = special
+    kc, vc = kc.to(dtype), vc.to(dtype)
+    gen = torch.Generator().manual_seed(9)
+    T = sum(n for _c, n in specs)
+    q = torch.randn(T, n_q, D, generator=gen).to(torch.bfloat16)
+    i32 = dict(dtype=torch.int32)
+    lens = torch.tensor([c + n for c, n in specs], **i32)
+    starts = torch.tensor([sum(n for _c, n in specs[:i])
+                           for i in range(len(specs))], **i32)
+    qlens = torch.tensor([n for _c, n in specs], **i32)
+    out = torch.zeros(T, n_q, D, dtype=torch.bfloat16, device=DEV)
+    ops.paged_prefill_attention(
+        out, q.to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), lens.to(DEV),
+        starts.to(DEV), qlens.to(DEV), 0.05, max_qlen=int(qlens.max()))
+    want = torch.zeros(T, n_q, D)
+    ref.paged_prefill_attention(want, q.float(), kc.float(), vc.float(),
+                                table, lens, starts, qlens, 0.05)
+    last = (starts + qlens - 1).long()
+    got, want = out.float().cpu(), want
+    assert torch.equal(got[:, :, 127].isfinite(), want[:, :, 127].isfinite())
+    got, want = got[last], want[last]
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    bound = 2.0 ** -8 * float(vc.float()[vc.float().isfinite()].abs().max())
+    assert (got - want).abs()[fine].max().item() <= bound
+
+
 def test_rope_append_decode_is_both_steps():
     """Rotation, append and attention in one call against the single ops;
     a padded row (no tokens) is left alone, dirty counters do not matter."""
