@@ -131,7 +131,9 @@ class MixtralMoE(torch.nn.Module):
                        or (self.ep_mode == "auto" and T >= self.a2a_min_tokens))
             if use_a2a:
                 return self.forward_a2a(h, ep_group)
+        # (its products write into slices, which autograd does not record)
         if (h.is_cuda and T >= self.SPARSE_MIN_TOKENS
+                and not torch.is_grad_enabled()
                 and self.n_local == self.cfg.n_experts <= ops.STREAM_EXPERTS
                 and T * self.top_k < 1 << 24):
             out = self._experts_sorted(h)

@@ -490,6 +490,26 @@ def test_sorted_experts_are_the_gathered_ones():
     assert _rel(out, want) < 2.0 ** -7  # both round gate, up and result
 
 
+def test_experts_of_a_prompt_under_autograd():
+    """With gradients recorded, 65 rows and more take the products that
+    autograd accepts, as they did before the rows were sorted."""
+    from agentainer_amd.models.mixtral import MIXTRAL_CONFIGS, MixtralMoE
+    cfg = MIXTRAL_CONFIGS["tiny-mixtral"]
+    torch.manual_seed(3)
+    with torch.device(DEV):
+        moe = MixtralMoE(cfg)
+        with torch.no_grad():
+            for p in moe.parameters():
+                p.normal_(0.0, 0.05)
+        h = torch.randn(70, cfg.hidden_size, dtype=torch.bfloat16)
+    out = moe(h)
+    assert out.requires_grad
+    with torch.no_grad():
+        want = moe(h)
+    assert not want.requires_grad
+    assert _rel(out, want) < 2.0 ** -7  # both round gate, up and result
+
+
 def test_attention_rows_off_alignment():
     """Query rows and outputs two bytes off a 16-byte boundary, and a row
     stride that is no multiple of one: the same values as aligned ones."""
