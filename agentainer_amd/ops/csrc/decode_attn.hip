@@ -496,7 +496,8 @@ void decode_attention_counted(torch::Tensor out, torch::Tensor q,
               arrived.numel() >= (long)B * n_kv);
   TORCH_CHECK(!packed || B <= PACKED_ROWS);
   const int ms = packed ? packed_groups(B) : 0;
-  TORCH_CHECK(out.numel() == (packed ? (long)ms * 16 : (long)B) * n_q * Dh);
+  const long out_size = (packed ? (long)ms * 16 : (long)B) * n_q * Dh;
+  TORCH_CHECK(packed ? out.numel() == out_size : out.numel() >= out_size);
   const long pairs = (long)B * n_kv;
   const int n_split = splits_of(pairs, (long)max_pages * PS);
   auto part = torch::empty(

@@ -451,11 +451,22 @@ void paged_prefill_attention(torch::Tensor out, torch::Tensor q,
   };
   if (q.stride(0) % 8 != 0 || !aligned(q))
     q = q.clone(at::MemoryFormat::Contiguous);
-  if (!aligned(out)) {
-    auto rows = out.clone();
+  const long t_rows = q.size(0);
+  TORCH_CHECK(!packed || t_rows <= PACKED_ROWS);
+  const int ms = packed ? packed_groups(t_rows) : 0;
+  const long out_size = (packed ? (long)ms * 16 : t_rows) * n_q * Dh;
+  TORCH_CHECK(!packed || out.numel() == out_size);
+  // more rows than q's are left alone; fewer are enough where the sequences
+  // cover no more
+  if (!aligned(out) || out.numel() < out_size) {
+    auto rows = torch::empty({out_size}, out.options());
+    auto all = out.view({-1});
+    const long n = std::min<long>(out_size, all.numel());
+    auto part = all.narrow(0, 0, n), mine = rows.narrow(0, 0, n);
+    mine.copy_(part);
     paged_prefill_attention(rows, q, k_cache, v_cache, page_table, seq_lens,
                             query_starts, query_lens, scale, max_qlen, packed);
-    out.copy_(rows);
+    part.copy_(mine);
     return;
   }
   const int qtiles = (max_qlen + QBLK - 1) / QBLK;
@@ -472,10 +483,6 @@ void paged_prefill_attention(torch::Tensor out, torch::Tensor q,
   if (blocks < 384)
     n_split = (int)std::max<long>(
         1, std::min<long>({16, 512 / blocks, ctx_tiles / 2}));
-  const long t_rows = q.size(0);
-  TORCH_CHECK(!packed || t_rows <= PACKED_ROWS);
-  const int ms = packed ? packed_groups(t_rows) : 0;
-  TORCH_CHECK(out.numel() == (packed ? (long)ms * 16 : t_rows) * n_q * Dh);
   torch::Tensor part;
   if (n_split > 1)
     part = torch::empty({n_split * t_rows * n_q * PART},

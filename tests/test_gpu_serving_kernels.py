@@ -652,3 +652,34 @@ def test_quantized_decode_is_row_major(name, quant, kv_dtype, T):
     ops.fused_add_rmsnorm(h, x, res, model.final_ln, eps)
     want = ops.linear(h, model.lm_head, model.lm_head_packed)
     assert torch.equal(got, want)
+
+
+def test_attention_outputs_of_other_sizes():
+    """An output with more rows than q keeps them; one with fewer than q
+    serves sequences that cover no more (prompts only)."""
+    n_q, n_kv, D, PS, lens = 8, 2, 128, 16, [40, 75, 9]
+    kc, vc, table = _paged(lens, n_kv, D, PS, torch.bfloat16, seed=2)
+    kc, vc, table = kc.to(DEV), vc.to(DEV), table.to(DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    B = len(lens)
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    q = torch.randn(B + 2, n_q, D, generator=gen, device=DEV).to(
+        torch.bfloat16)
+    new = lambda n: torch.full((n, n_q, D), 7.0, dtype=torch.bfloat16,  # noqa: E731
+                               device=DEV)
+    want, more = new(B), new(B + 3)
+    ops.paged_decode_attention(want, q[:B], kc, vc, table, sl, 0.1)
+    ops.paged_decode_attention(more, q[:B], kc, vc, table, sl, 0.1)
+    assert torch.equal(more[:B], want) and bool((more[B:] == 7.0).all())
+    with pytest.raises(RuntimeError):
+        ops.paged_decode_attention(new(B - 1), q[:B], kc, vc, table, sl, 0.1)
+    starts = torch.arange(B, dtype=torch.int32, device=DEV)
+    ones = torch.ones(B, dtype=torch.int32, device=DEV)
+    for tb in (table, torch.nn.functional.pad(table, (0, 64))):  # split runs
+        args = (kc, vc, tb, sl, starts, ones, 0.1)
+        want, more, fewer = new(B), new(B + 4), new(B)
+        ops.paged_prefill_attention(want, q[:B], *args, max_qlen=1)
+        ops.paged_prefill_attention(more, q[:B], *args, max_qlen=1)
+        ops.paged_prefill_attention(fewer, q, *args, max_qlen=1)
+        assert torch.equal(more[:B], want) and bool((more[B:] == 7.0).all())
+        assert torch.equal(fewer, want)
