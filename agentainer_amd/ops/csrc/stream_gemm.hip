@@ -542,7 +542,7 @@ void stream_gemm_experts(torch::Tensor out, torch::Tensor x,
   TORCH_CHECK(experts >= 1 && experts <= MAX_EXPERTS);
   TORCH_CHECK(T <= 64 && T * top_k <= MAX_PAIRS);
   TORCH_CHECK(mode == PARTS || mode == SILU);
-  TORCH_CHECK(N % 64 == 0 && K % FRAG_K == 0);
+  TORCH_CHECK(N % (mode == SILU ? 64 : 32) == 0 && K % FRAG_K == 0);
   const int rows = mode == SILU ? T : T * top_k;
   const int x_groups = mode == SILU ? packed_groups(T) : (rows + 15) / 16;
   const int pair_groups = (T * top_k + 15) / 16;

@@ -683,3 +683,87 @@ def test_attention_outputs_of_other_sizes():
         ops.paged_prefill_attention(fewer, q, *args, max_qlen=1)
         assert torch.equal(more[:B], want) and bool((more[B:] == 7.0).all())
         assert torch.equal(fewer, want)
+
+
+def _prefill_state(cfg, specs, seed, PS=16):
+    """Caches, metadata, tokens and last rows of a prompt step of (cached,
+    new) tokens per sequence."""
+    from agentainer_amd.models.llama import AttnMetadata
+    lens = [c + n for c, n in specs]
+    caches = []
+    for i in range(cfg.n_layers):
+        kc, vc, table = _paged(lens, cfg.n_kv_heads, cfg.head_dim, PS,
+                               torch.bfloat16, seed=seed)
+        caches.append((kc.nan_to_num().to(DEV), vc.nan_to_num().to(DEV)))
+    pos = torch.cat([torch.arange(c, c + n) for c, n in specs])
+    seq = torch.repeat_interleave(torch.arange(len(specs)),
+                                  torch.tensor([n for _c, n in specs]))
+    slots = table[seq, pos // PS].long() * PS + pos % PS
+    i32 = dict(dtype=torch.int32, device=DEV)
+    starts = [sum(n for _c, n in specs[:i]) for i in range(len(specs))]
+    md = AttnMetadata(
+        page_table=table.to(DEV), seq_lens=torch.tensor(lens, **i32),
+        slot_mapping=slots.to(DEV), positions=pos.to(torch.int32).to(DEV),
+        is_prefill=True, query_starts=torch.tensor(starts, **i32),
+        query_lens=torch.tensor([n for _c, n in specs], **i32),
+        max_qlen=max(n for _c, n in specs))
+    gen = torch.Generator().manual_seed(seed)
+    ids = torch.randint(0, cfg.vocab_size, (len(pos),), generator=gen)
+    last = torch.tensor([s + n - 1 for s, (_c, n) in zip(starts, specs)])
+    return caches, md, ids.to(DEV), last.to(DEV)
+
+
+@pytest.mark.parametrize("family,change", [
+    ("llama", {}),
+    ("llama", {"qkv_bias": True, "n_heads": 8, "n_kv_heads": 2}),
+    ("llama", {"hidden_size": 96, "intermediate_size": 160,
+               "vocab_size": 352}),
+    ("mixtral", {}),
+    # a hidden size of whole fragments, but not of pairs of them
+    ("mixtral", {"hidden_size": 96, "intermediate_size": 160}),
+])
+@pytest.mark.parametrize("T", [1, 17, 64, 65, 128])
+@pytest.mark.parametrize("prompt", [False, True])
+@torch.no_grad()
+def test_streamed_forward_is_the_row_major_one(family, change, T, prompt):
+    """The whole step over packed weights and rows against the same model's
+    row-major forward."""
+    from dataclasses import replace
+    from agentainer_amd.models import llama, mixtral
+    if family == "llama":
+        cfg = replace(llama.LLAMA_CONFIGS["tiny-llama"], **change)
+        model = llama.LlamaForCausalLM(cfg, DEV)
+    else:
+        cfg = replace(mixtral.MIXTRAL_CONFIGS["tiny-mixtral"], **change)
+        model = mixtral.MixtralForCausalLM(cfg, DEV)
+        # a clear choice of experts: bf16 and fp32 logits choose alike
+        for layer in model.layers:
+            layer.moe.router.normal_(0.0, 1.0)
+    if cfg.qkv_bias:
+        for layer in model.layers:
+            layer.attn.qkv_bias.normal_(0.0, 0.5)
+    model.pack_decode_weights()
+    if prompt:
+        specs = ([(40, T)] if T < 3 else
+                 [(0, T // 3), (33, 1), (16, T - T // 3 - 1)])
+        caches, md, ids, last = _prefill_state(cfg, specs, T)
+    else:
+        caches, md, ids = _decode_state(
+            cfg, [5 + 7 * i for i in range(T)], torch.bfloat16, cfg.n_layers,
+            T)
+        last = None
+    copies = [(k.clone(), v.clone()) for k, v in caches]
+    streams = llama.can_stream(model, ids)
+    assert streams == (family == "llama" or T <= ops.STREAM_ROWS)
+    got = model(ids, md, caches, last)
+    head, model.lm_head_packed = model.lm_head_packed, None
+    assert not llama.can_stream(model, ids)
+    want = model(ids, md, copies, last)
+    assert got.shape == want.shape
+    # some 20 bf16 roundings in a row in either, 2^-9 of a value each
+    err = (got.float() - want.float()).norm(dim=1) / want.float().norm(dim=1)
+    if family == "mixtral":  # a token near a tie may take another expert
+        err = err.sort().values[:max(1, T * 9 // 10)]
+    assert err.max().item() < 2.0 ** -5
+    for (k0, v0), (k1, v1) in zip(caches, copies):
+        assert _rel(k0, k1) < 2.0 ** -6 and _rel(v0, v1) < 2.0 ** -6
