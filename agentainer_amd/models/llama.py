@@ -290,6 +290,7 @@ def can_stream(model, input_ids) -> bool:
     T = input_ids.numel()
     return (input_ids.is_cuda and 0 < T <= ops.STREAM_ROWS_WIDE
             and model.tp_group is None
+            and not (ops.SKINNY_DISABLED or ops.SKINNY_FORCED)
             and getattr(model, "lm_head_packed", None) is not None
             and model.lm_head.size(0) % 32 == 0
             and model.cfg.hidden_size % 32 == 0

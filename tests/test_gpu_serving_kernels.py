@@ -685,6 +685,26 @@ def test_attention_outputs_of_other_sizes():
         assert torch.equal(fewer, want)
 
 
+@pytest.mark.parametrize("switch", ["SKINNY_DISABLED", "SKINNY_FORCED"])
+@torch.no_grad()
+def test_projection_switches_reach_the_whole_step(switch, monkeypatch):
+    """The switches that choose a projection's kernel choose it for decode
+    steps too: none of them streams then."""
+    from agentainer_amd.models import llama
+    cfg = llama.LLAMA_CONFIGS["tiny-llama"]
+    model = llama.LlamaForCausalLM(cfg, DEV)
+    model.pack_decode_weights()
+    caches, md, ids = _decode_state(cfg, [9, 30, 2], torch.bfloat16,
+                                    cfg.n_layers, 1)
+    monkeypatch.setattr(ops, switch, True)
+    streamed = []
+    for name in ("stream_linear", "stream_parts", "stream_gate_up"):
+        monkeypatch.setattr(ops, name, lambda *a, n=name, **k:
+                            streamed.append(n))
+    logits = model(ids, md, caches)
+    assert logits.isfinite().all() and not streamed
+
+
 def _prefill_state(cfg, specs, seed, PS=16):
     """Caches, metadata, tokens and last rows of a prompt step of (cached,
     new) tokens per sequence."""
