@@ -1096,7 +1096,10 @@ class ModelInstance:
         ids_pin = torch.zeros(bucket, dtype=torch.long, pin_memory=self.is_gpu)
         entry = {"rows": rows, "ids": ids, "inc": inc, "rows_pin": rows_pin,
                  "ids_pin": ids_pin, "graph": None, "logits": None}
-        if self.use_graph:
+        # a model may know sizes whose step waits for the host: those buckets
+        # run eagerly, the others keep their graphs
+        captures = getattr(self.model, "captures", None)
+        if self.use_graph and (captures is None or captures(bucket)):
             try:
                 for _ in range(2):  # warmup before capture (also exercises
                     self._device_decode_fwd(rows, ids, inc)  # RCCL comms)

@@ -431,6 +431,11 @@ class MixtralForCausalLM(torch.nn.Module):
                         layer.moe.down[i].data)
         self.lm_head_packed = ops.pack_weight(self.lm_head.data)
 
+    def captures(self, rows: int) -> bool:
+        """Whether a decode step of so many rows can be captured: from
+        SPARSE_MIN_TOKENS on the host waits for the experts' row counts."""
+        return rows < MixtralMoE.SPARSE_MIN_TOKENS
+
     @torch.no_grad()
     def forward(self, input_ids, md: AttnMetadata, kv_caches,
                 last_rows=None) -> torch.Tensor:

@@ -705,6 +705,35 @@ def test_projection_switches_reach_the_whole_step(switch, monkeypatch):
     assert logits.isfinite().all() and not streamed
 
 
+def test_large_expert_batches_leave_the_graphs_on():
+    """A decode batch of a mixture above the captured sizes runs eagerly, by
+    itself: smaller ones are still captured, also after it."""
+    from agentainer_amd.engine.llm import ModelInstance
+    from agentainer_amd.models.mixtral import (MIXTRAL_CONFIGS,
+                                               MixtralForCausalLM)
+    cfg = MIXTRAL_CONFIGS["tiny-mixtral"]
+
+    def step(graph):
+        inst = ModelInstance("tiny-mixtral", cfg, DEV,
+                             {"sync_mode": True, "kv_pool_tokens": 4096,
+                              "graph_capture": graph},
+                             model_cls=MixtralForCausalLM)
+        ids = [("a%d" % i, [3 + i, 7, 11 + i]) for i in range(70)]
+        inst.forward_step(ids, [[2]] * 70)
+        large = inst.forward_step([(s, [5 + i]) for i, (s, _t)
+                                   in enumerate(ids)], [[0]] * 70)
+        large = large.clone()
+        return inst, large, inst.forward_step([(s, [9]) for s, _t in ids[:3]],
+                                              [[0]] * 3)
+
+    inst, large, small = step(True)
+    assert inst.use_graph
+    assert inst._graphs[128]["graph"] is None
+    assert inst._graphs[4]["graph"] is not None
+    _plain, large0, small0 = step(False)
+    assert torch.equal(large, large0) and torch.equal(small, small0)
+
+
 def _prefill_state(cfg, specs, seed, PS=16):
     """Caches, metadata, tokens and last rows of a prompt step of (cached,
     new) tokens per sequence."""
