@@ -490,6 +490,36 @@ def test_sorted_experts_are_the_gathered_ones():
     assert _rel(out, want) < 2.0 ** -7  # both round gate, up and result
 
 
+def test_sorted_experts_in_groups(monkeypatch):
+    """Groups of experts: the same bits as all at once, and less memory
+    between gate and down."""
+    from agentainer_amd.models.mixtral import MIXTRAL_CONFIGS, MixtralMoE
+    cfg = MIXTRAL_CONFIGS["tiny-mixtral"]
+    torch.manual_seed(4)
+    with torch.device(DEV), torch.no_grad():
+        moe = MixtralMoE(cfg)
+        for p in moe.parameters():
+            p.normal_(0.0, 0.05)
+        h = torch.randn(5000, cfg.hidden_size, dtype=torch.bfloat16)
+
+        def peak():
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            base = torch.cuda.memory_allocated()
+            out = moe(h)
+            torch.cuda.synchronize()
+            return out, torch.cuda.max_memory_allocated() - base
+
+        moe(h)  # the library's workspaces
+        out, used = peak()
+        monkeypatch.setattr(MixtralMoE, "SORTED_PAIRS", 1 << 30)
+        want, used_at_once = peak()
+    assert torch.equal(out, want)
+    # 3 * inter columns of bf16 for 10000 pairs against at most 4096 (or one
+    # expert's, of four)
+    assert used < used_at_once - 3 * cfg.intermediate_size * 2 * 2000
+
+
 def test_experts_of_a_prompt_under_autograd():
     """With gradients recorded, 65 rows and more take the products that
     autograd accepts, as they did before the rows were sorted."""
