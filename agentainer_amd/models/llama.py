@@ -144,15 +144,14 @@ class LlamaAttention(torch.nn.Module):
         return self.qkv_packed, self.o_packed
 
     def forward_packed(self, x, T, k_cache, v_cache, md, cos_sin):
-        """Packed rows in (row-major above ops.STREAM_ROWS, where the fused
-        projection has too few column tiles to stream), fp32 parts of the
-        residual update out."""
+        """Rows in (packed where the fused projection streams them, see
+        ops.streams), fp32 parts of the residual update out."""
         hid = self.cfg.hidden_size
         w_qkv, w_o = self.stream_weights()
-        if T > ops.STREAM_ROWS:
-            qkv = ops.linear(x, self.qkv_proj)
-        else:
+        if ops.streams(T, self.qkv_proj.size(0)):
             qkv = ops.stream_linear(x, T, w_qkv, self.qkv_proj.size(0), hid)
+        else:
+            qkv = ops.linear(x, self.qkv_proj)
         if self.qkv_bias is not None:
             qkv = qkv + self.qkv_bias
         o = self.attend(qkv, k_cache, v_cache, md, cos_sin, packed=True)
@@ -198,10 +197,17 @@ class LlamaMLP(torch.nn.Module):
         return self.gate_up_packed, self.down_packed
 
     def forward_packed(self, x, T):
-        """Packed rows in, fp32 parts of the residual update out."""
+        """Rows in (packed where gate and up stream them), fp32 parts of the
+        residual update out."""
         hid = self.down.size(0)
         w_gate_up, w_down = self.stream_weights()
-        act = ops.stream_gate_up(x, T, w_gate_up, 2 * self.inter, hid)
+        if ops.streams(T, 2 * self.inter):
+            act = ops.stream_gate_up(x, T, w_gate_up, 2 * self.inter, hid)
+        else:
+            gu = ops.linear(x, self.gate_up)
+            act = torch.empty(T, self.inter, dtype=gu.dtype, device=gu.device)
+            ops.silu_mul(act, gu[:, :self.inter], gu[:, self.inter:])
+            act = ops.pack_rows(act)
         return ops.stream_parts(act, T, w_down, hid, self.inter)
 
     def forward(self, h, tp_group=None):
@@ -249,16 +255,20 @@ class LlamaLayer(torch.nn.Module):
     def streams(self, T):
         """Whether forward_packed can take T rows."""
         return (self.attn.stream_weights() is not None
-                and self.mlp.stream_weights() is not None)
+                and self.mlp.stream_weights() is not None
+                and (ops.streams(T, 2 * self.mlp.inter)
+                     or ops.streams_parts(T, self.attn.cfg.hidden_size)))
 
     def forward_packed(self, parts, residual, k_cache, v_cache, md, cos_sin):
         """At most ops.STREAM_ROWS_WIDE rows: `parts` (None in the first layer) is
         what the layer before still has to add to the residual."""
         T = residual.size(0)
         x = ops.add_parts_rmsnorm(residual, parts, self.input_ln, self.eps,
-                                  packed=T <= ops.STREAM_ROWS)
+                                  packed=ops.streams(
+                                      T, self.attn.qkv_proj.size(0)))
         parts = self.attn.forward_packed(x, T, k_cache, v_cache, md, cos_sin)
-        x = ops.add_parts_rmsnorm(residual, parts, self.post_ln, self.eps)
+        x = ops.add_parts_rmsnorm(residual, parts, self.post_ln, self.eps,
+                                  packed=ops.streams(T, 2 * self.mlp.inter))
         return self.mlp.forward_packed(x, T)
 
 
@@ -271,16 +281,19 @@ def forward_streamed(model, input_ids, md, kv_caches, last_rows):
     for layer, (k_cache, v_cache) in zip(model.layers, kv_caches):
         parts = layer.forward_packed(parts, residual, k_cache, v_cache, md,
                                      model.cos_sin)
+    vocab = model.lm_head.size(0)
+    packed = last_rows is None and ops.streams(T, vocab)
     x = ops.add_parts_rmsnorm(residual, parts, model.final_ln,
-                              model.cfg.norm_eps, packed=last_rows is None)
+                              model.cfg.norm_eps, packed=packed)
     if last_rows is not None:
         x = x[last_rows]
         T = x.size(0)
-        if T > ops.STREAM_ROWS_WIDE:
-            return ops.linear(x, model.lm_head, model.lm_head_packed)
-        x = ops.pack_rows(x)
-    return ops.stream_linear(x, T, model.lm_head_packed,
-                             model.lm_head.size(0), hid)
+        packed = T <= ops.STREAM_ROWS_WIDE and ops.streams(T, vocab)
+        if packed:
+            x = ops.pack_rows(x)
+    if not packed:
+        return ops.linear(x, model.lm_head, model.lm_head_packed)
+    return ops.stream_linear(x, T, model.lm_head_packed, vocab, hid)
 
 
 def can_stream(model, input_ids) -> bool:

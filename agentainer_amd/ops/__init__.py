@@ -293,7 +293,34 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 # partial sums [splits, T, N] that add_parts_rmsnorm adds up.
 
 STREAM_ROWS = 64         # every projection of a layer, and experts
-STREAM_ROWS_WIDE = 128   # projections with many column tiles
+STREAM_ROWS_WIDE = 128   # projections that streams() or streams_parts() names
+# From 65 rows on a workgroup takes 128 columns, and a projection needs some
+# 160 of them to outrun the library: us for 80 / 128 rows, streamed against
+# library (with its silu), cold weights of N x K
+#   16384 x 2048  28.8 / 29.2 against 23.3 / 25.2    (128 workgroups)
+#   16384 x 4096  55.5 / 56.0 against 39.9 / 41.9
+#   10240 x 8192   103 / 104  against 76.0 / 58.2    (80)
+#   28672 x 2048  32.3 / 33.0 against 44.5 / 36.7    (224)
+#   28672 x 4096  66.6 / 66.7 against 71.7 / 60.0
+#   57344 x 8192   196 / 197  against  185 / 206     (448)
+STREAM_WIDE_N = 20480
+# Projections into the residual split K by up to 8 and save the library its
+# extra pass; with the norm behind both:
+#    2048 x 5632  19.3 / 21.3 against 19.1 / 19.4
+#    3072 x 8192  25.7 / 26.7 against 42.7 / 45.2
+#    4096 x 14336 41.2 / 43.2 against 47.5 / 79.4
+STREAM_PARTS_N = 3072
+
+
+def streams(T: int, N: int) -> bool:
+    """Whether T packed rows are projected to N columns faster than row-major
+    ones by the library."""
+    return T <= STREAM_ROWS or N >= STREAM_WIDE_N
+
+
+def streams_parts(T: int, N: int) -> bool:
+    """The same for projections into a residual stream of N columns."""
+    return T <= STREAM_ROWS or N >= STREAM_PARTS_N
 
 
 def packed_rows(T: int, K: int, device) -> torch.Tensor:

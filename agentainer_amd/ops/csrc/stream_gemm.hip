@@ -330,8 +330,8 @@ void dispatch_grouped(const StreamArgs& a, const Weights<true>& w, int mode,
 //   o        4096 x 4096  14 (24)    lm_head           210 (234)
 //   8192 x 28672          94 (200)   8192 x 8192        32 (48)
 // A projection that is neither split nor large (qkv: 48 workgroups, 52 us
-// against 26) is left to the library, and so are more than 128 rows, where
-// twice the x makes gate_up 81 us against 70.
+// against 26) is left to the library (ops.streams has the line), and so are
+// more than 128 rows, where twice the x makes gate_up 81 us against 70.
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(
     void* __restrict__ out, const char* __restrict__ x,

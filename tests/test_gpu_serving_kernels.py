@@ -797,6 +797,12 @@ def _prefill_state(cfg, specs, seed, PS=16):
     ("llama", {"qkv_bias": True, "n_heads": 8, "n_kv_heads": 2}),
     ("llama", {"hidden_size": 96, "intermediate_size": 160,
                "vocab_size": 352}),
+    # above 64 rows: gate and up by the library, the residual's parts streamed
+    ("llama", {"hidden_size": 3072, "intermediate_size": 512}),
+    # ... gate and up streamed, and the last projection
+    ("llama", {"intermediate_size": 10240, "vocab_size": 20480}),
+    # ... and the fused one
+    ("llama", {"n_heads": 128, "n_kv_heads": 16, "hidden_size": 3072}),
     ("mixtral", {}),
     # a hidden size of whole fragments, but not of pairs of them
     ("mixtral", {"hidden_size": 96, "intermediate_size": 160}),
@@ -833,7 +839,8 @@ def test_streamed_forward_is_the_row_major_one(family, change, T, prompt):
         last = None
     copies = [(k.clone(), v.clone()) for k, v in caches]
     streams = llama.can_stream(model, ids)
-    assert streams == (family == "llama" or T <= ops.STREAM_ROWS)
+    assert streams == (T <= 64 or family == "llama" and (
+        cfg.hidden_size >= 3072 or cfg.intermediate_size >= 10240))
     got = model(ids, md, caches, last)
     head, model.lm_head_packed = model.lm_head_packed, None
     assert not llama.can_stream(model, ids)
