@@ -198,7 +198,6 @@ def topp_sample(out, logits, temps, top_ps, seeds):
     return out
 
 
-_ws_cache = {}
 _EMPTY_WS = {}
 SKINNY_DISABLED = os.environ.get("AGENTAINER_DISABLE_SKINNY", "0") == "1"
 SKINNY_FORCED = os.environ.get("AGENTAINER_FORCE_SKINNY", "0") == "1"
@@ -239,13 +238,10 @@ def pack_weight(w: torch.Tensor) -> torch.Tensor:
 
 
 def _skinny_ws(device, N: int, split: int) -> torch.Tensor:
+    """fp32 parts of one call's split K. Not kept: a prompt step on its own
+    stream and a decode step run the same projection at the same time."""
     if split > 1:
-        key = (device, N, split)
-        ws = _ws_cache.get(key)
-        if ws is None or ws.numel() < split * 64 * N:
-            ws = torch.empty(split * 64 * N, dtype=torch.float32, device=device)
-            _ws_cache[key] = ws
-        return ws
+        return torch.empty(split * 64 * N, dtype=torch.float32, device=device)
     ws = _EMPTY_WS.get(device)
     if ws is None:
         ws = torch.empty(1, dtype=torch.float32, device=device)

@@ -200,6 +200,14 @@ def test_mxfp4_pack_roundtrip():
     assert torch.equal(ops.dequantize_mxfp4(p2, s2, 16, 128), w2.float())
 
 
+def test_split_workspaces_are_not_shared():
+    """Two projections in flight (a prompt step beside a decode step) never
+    sum in the same memory."""
+    a = ops._skinny_ws(torch.device("cpu"), 128, 4)
+    b = ops._skinny_ws(torch.device("cpu"), 128, 4)
+    assert a.numel() >= 4 * 64 * 128 and a.data_ptr() != b.data_ptr()
+
+
 def test_linear_quant_dispatch_kinds():
     """linear_quant routes by kind tag; CPU tensors raise loudly (these
     paths are GPU-only by policy — no silent eager fallback)."""
