@@ -853,3 +853,66 @@ def test_streamed_forward_is_the_row_major_one(family, change, T, prompt):
     assert err.max().item() < 2.0 ** -5
     for (k0, v0), (k1, v1) in zip(caches, copies):
         assert _rel(k0, k1) < 2.0 ** -6 and _rel(v0, v1) < 2.0 ** -6
+
+
+def _codes(x, kind):
+    """What a row-quantized activation holds of bf16 rows x, in 64 bits."""
+    top = 448.0 if kind == "fp8" else 6.0
+    step = x.float().abs().amax(1, keepdim=True).clamp(min=1e-8) / top
+    y = x.float() * (1.0 / step)
+    if kind == "fp8":
+        q = y.to(torch.float8_e4m3fn).double()
+    else:
+        grid = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0],
+                            dtype=torch.float64)
+        mids = torch.tensor([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0])
+        # a magnitude on a midpoint takes the larger code
+        q = grid[torch.bucketize(y.abs(), mids, right=True)]
+        q = torch.where(y < 0, -q, q)
+    return q * step.double()
+
+
+@pytest.mark.parametrize("kind", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("T", [1, 13, 64])
+@torch.no_grad()
+def test_quantized_experts_against_their_codes(kind, T):
+    """A whole mixture layer against 64-bit products of the codes that its
+    weights and activations are stored in."""
+    from agentainer_amd.models.mixtral import (MIXTRAL_CONFIGS,
+                                               MixtralForCausalLM)
+    cfg = MIXTRAL_CONFIGS["tiny-mixtral"]
+    model = MixtralForCausalLM(cfg, DEV)
+    model.pack_decode_weights(expert_fp8=kind == "fp8",
+                              expert_fp4=kind == "mxfp4")
+    moe = model.layers[1].moe
+    gen = torch.Generator().manual_seed(T)
+    moe.router.copy_(torch.randn(moe.router.shape, generator=gen))
+    h = torch.randn(T, cfg.hidden_size, generator=gen).to(torch.bfloat16)
+    got = moe(h.to(DEV)).double().cpu()
+
+    bf = lambda x: x.to(torch.bfloat16).double()  # noqa: E731
+    def weight(w):
+        N, K = w.shape
+        if kind == "mxfp4":
+            p, sc = ops.quantize_weight_mxfp4(w)
+            return ops.dequantize_mxfp4(p, sc, N, K).double()
+        p, sc = ops.quantize_weight_fp8(w)
+        q = p.cpu().view(torch.float8_e4m3fn).double().view(
+            N // 16, K // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(N, K)
+        return q * sc.cpu().double()[:, None]
+
+    # the layer's own bf16 logits: a step of one of them is 0.125
+    logits = torch.nn.functional.linear(h.to(DEV), moe.router).double().cpu()
+    top, who = torch.softmax(logits, -1).topk(cfg.top_k, -1)
+    top = top / top.sum(-1, keepdim=True)
+    want = torch.zeros(T, cfg.hidden_size, dtype=torch.float64)
+    x = _codes(h, kind)
+    for e in range(cfg.n_experts):
+        g, u = bf(x @ weight(moe.gate_up[e]).t()).chunk(2, dim=1)
+        act = (g / (1.0 + torch.exp(-g)) * u).to(torch.bfloat16)
+        y = bf(_codes(act, kind) @ weight(moe.down[e]).t())
+        want += torch.where(who == e, top, torch.zeros_like(top)).sum(
+            -1, keepdim=True) * y
+    # the result's rounding (2^-9), and one activation in some thousands that
+    # rounds to the other neighbour and may change its code
+    assert ((got - want).norm() / want.norm()).item() < 2.0 ** -7
