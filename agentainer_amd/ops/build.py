@@ -96,6 +96,11 @@ def _newest(paths):
     return max(os.path.getmtime(p) for p in paths if os.path.exists(p))
 
 
+def _headers():
+    return [os.path.join(CSRC, f) for f in sorted(os.listdir(CSRC))
+            if f.endswith(".h")]
+
+
 def _target(target: str):
     """(output .so, object dir, sources, module name) of a build target."""
     if target == "latent":
@@ -128,9 +133,7 @@ def needs_build(target: str = "core") -> bool:
     if not os.path.exists(OUT):
         return True
     srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    srcs.append(os.path.join(CSRC, "common.h"))
-    srcs.append(os.path.join(CSRC, "latent_common.h"))
-    srcs.append(os.path.join(CSRC, "matrix_memory_kernel.h"))
+    srcs += _headers()
     srcs.append(os.path.abspath(__file__))
     return _newest(srcs) > os.path.getmtime(OUT)
 
@@ -170,9 +173,7 @@ def build(verbose: bool = True, force: bool = False,
         objs.append(obj)
         if (os.path.exists(obj)
                 and os.path.getmtime(obj) > _newest(
-                    [src_path, os.path.join(CSRC, "common.h"),
-                     os.path.join(CSRC, "latent_common.h"),
-                     os.path.join(CSRC, "matrix_memory_kernel.h")])
+                    [src_path] + _headers())
                 and not force):
             continue
         san = (["-fsanitize=address", "-shared-libsan"]

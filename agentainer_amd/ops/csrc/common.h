@@ -89,26 +89,12 @@ __device__ __forceinline__ void fp8x8_to_f32(const u8x8 v, float* out) {
   out[4] = p2.x; out[5] = p2.y; out[6] = p3.x; out[7] = p3.y;
 }
 
-// e2m1 encode: nearest of {0,.5,1,1.5,2,3,4,6} with sign bit 3
-__device__ __forceinline__ unsigned char f2e2m1(float v) {
-  const float a = fabsf(v);
-  unsigned char c;
-  if (a < 0.25f) c = 0;
-  else if (a < 0.75f) c = 1;
-  else if (a < 1.25f) c = 2;
-  else if (a < 1.75f) c = 3;
-  else if (a < 2.5f) c = 4;
-  else if (a < 3.5f) c = 5;
-  else if (a < 5.0f) c = 6;
-  else c = 7;
-  return c | (v < 0.f ? 8 : 0);
-}
-
 // Rows of a step (M <= 128) packed for the streaming projections: the
 // 16 x 32 fragments an MFMA takes, [k / 32][row / 16][lane][8], 1 KB each. ms
-// is the number of 16-row groups (a power of two up to 8). Row-major rows are what the
-// projections cannot read fast: a fragment then is 16 pieces of 64 bytes, one
-// row stride apart, which meet in one memory channel.
+// is the number of 16-row groups: a power of two up to 8 for the rows of a
+// step, (pairs + 15) / 16 for the pairs that experts work on. Row-major rows
+// are what the projections cannot read fast: a fragment then is 16 pieces of
+// 64 bytes, one row stride apart, which meet in one memory channel.
 __device__ __forceinline__ long packed_at(int row, int k, int ms) {
   return ((long)(k / 32) * ms + row / 16) * 512 +
          ((k % 32) / 8 * 16 + row % 16) * 8 + k % 8;

@@ -11,62 +11,9 @@
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
-#include "common.h"
+#include "expert_route.h"
 
 namespace {
-
-constexpr int MAX_EXPERTS = 16;
-
-// One token per workgroup: fp32 logits of E experts, the top_k largest (lowest
-// index first among equals), softmax weights over the chosen ones.
-__global__ __launch_bounds__(256) void route_rows_kernel(
-    int* __restrict__ choice, float* __restrict__ weight,
-    const short* __restrict__ x, const short* __restrict__ router, int K,
-    int E, int top_k) {
-  const long row = blockIdx.x;
-  float acc[MAX_EXPERTS];
-#pragma unroll
-  for (int e = 0; e < MAX_EXPERTS; ++e) acc[e] = 0.f;
-  for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
-    const bf16x8 v = *reinterpret_cast<const bf16x8*>(x + row * K + k);
-#pragma unroll
-    for (int e = 0; e < MAX_EXPERTS; ++e) {
-      if (e >= E) break;
-      const bf16x8 r =
-          *reinterpret_cast<const bf16x8*>(router + (long)e * K + k);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        acc[e] = fmaf(bits2f(v[j]), bits2f(r[j]), acc[e]);
-    }
-  }
-  __shared__ float red[4][MAX_EXPERTS];
-#pragma unroll
-  for (int e = 0; e < MAX_EXPERTS; ++e) {
-    if (e >= E) break;
-    const float s = wave_sum(acc[e]);
-    if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE][e] = s;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  float logit[MAX_EXPERTS], mx = -INFINITY;
-  for (int e = 0; e < E; ++e) {
-    logit[e] = red[0][e] + red[1][e] + red[2][e] + red[3][e];
-    mx = fmaxf(mx, logit[e]);
-  }
-  unsigned taken = 0;
-  float sum = 0.f;
-  for (int i = 0; i < top_k; ++i) {
-    int best = -1;
-    for (int e = 0; e < E; ++e)
-      if (!(taken >> e & 1) && (best < 0 || logit[e] > logit[best])) best = e;
-    taken |= 1u << best;
-    choice[row * top_k + i] = best;
-    const float p = __expf(logit[best] - mx);
-    weight[row * top_k + i] = p;
-    sum += p;
-  }
-  for (int i = 0; i < top_k; ++i) weight[row * top_k + i] /= sum;
-}
 
 // Workgroup e: the pairs that chose expert e, in order, behind those of the
 // experts below it. place[pair] is where the pair's row goes.
@@ -170,10 +117,10 @@ void route_rows(torch::Tensor choice, torch::Tensor weight, torch::Tensor order,
               weight.numel() == choice.numel());
   if (T == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(route_rows_kernel, dim3(T), dim3(256), 0, stream,
+  hipLaunchKernelGGL(route_kernel<false>, dim3(T), dim3(256), 0, stream,
                      choice.data_ptr<int>(), weight.data_ptr<float>(),
                      (const short*)x.data_ptr(), (const short*)router.data_ptr(),
-                     K, E, top_k);
+                     K, 0, E, top_k);
   hipLaunchKernelGGL(sort_pairs_kernel, dim3(E), dim3(256), 0, stream,
                      order.data_ptr<int>(), place.data_ptr<int>(),
                      counts.data_ptr<int>(), choice.data_ptr<int>(),

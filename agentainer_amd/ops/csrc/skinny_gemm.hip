@@ -556,6 +556,21 @@ __global__ __launch_bounds__(256) void skinny_gemm_fp8_kernel(
 
 namespace {
 
+// e2m1 encode: nearest of {0,.5,1,1.5,2,3,4,6} with sign bit 3
+__device__ __forceinline__ unsigned char f2e2m1(float v) {
+  const float a = fabsf(v);
+  unsigned char c;
+  if (a < 0.25f) c = 0;
+  else if (a < 0.75f) c = 1;
+  else if (a < 1.25f) c = 2;
+  else if (a < 1.75f) c = 3;
+  else if (a < 2.5f) c = 4;
+  else if (a < 3.5f) c = 5;
+  else if (a < 5.0f) c = 6;
+  else c = 7;
+  return c | (v < 0.f ? 8 : 0);
+}
+
 // per-row dynamic fp4 quantization: x bf16 [M,K] -> x4 [M,K/2] (2 codes
 // per byte, lo nibble = even k) + sx f32 [M] with amax -> 6.0
 __global__ __launch_bounds__(256) void quant_fp4_rows_kernel(

@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <vector>
 #include "common.h"
+#include "expert_route.h"
 
 namespace {
 
@@ -41,7 +42,6 @@ typedef __bf16 bf16v4 __attribute__((ext_vector_type(4)));
 typedef int i32x4v __attribute__((ext_vector_type(4)));
 
 enum Mode { BF16 = 0, PARTS = 1, SILU = 2 };
-constexpr int MAX_EXPERTS = 16;
 constexpr int MAX_PAIRS = 128;
 
 constexpr int FRAG_K = 32;           // k per fragment
@@ -473,8 +473,8 @@ void check_packed(const torch::Tensor& x, long groups, long K) {
 
 }  // namespace
 
-// Splits of K that keep two workgroups' worth of tiles on every CU: N = 4096
-// (128 workgroups of two tiles) takes 2, N >= 8192 fills the chip alone. Above
+// Splits of K that give every CU a workgroup: N = 4096 (128 workgroups of two
+// tiles) takes 2, N >= 8192 has 256 and fills the chip alone. Above
 // 64 rows a workgroup has eight tiles and one stage's latency to hide (4096 x
 // 4096 at 128 rows: 51 us unsplit, 29, 18 and 14 in 2, 4 and 8).
 long stream_splits(long M, long N, long K) {
@@ -703,66 +703,6 @@ void pack_rows(torch::Tensor out, torch::Tensor x) {
                      (long)x.stride(0), n8);
 }
 
-// ---------------------------------------------------------------------------
-// The router.
-
-namespace {
-
-// Router of one token per workgroup: fp32 logits of E experts, softmax, the
-// top_k largest (lowest index first among equals), weights that sum to 1.
-__global__ __launch_bounds__(256) void route_packed_kernel(
-    int* __restrict__ choice, float* __restrict__ weight,
-    const short* __restrict__ x, const short* __restrict__ router, int K,
-    int groups, int E, int top_k) {
-  const int row = blockIdx.x;
-  float acc[MAX_EXPERTS];
-#pragma unroll
-  for (int e = 0; e < MAX_EXPERTS; ++e) acc[e] = 0.f;
-  for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
-    const bf16x8 v =
-        *reinterpret_cast<const bf16x8*>(x + packed_at(row, k, groups));
-#pragma unroll
-    for (int e = 0; e < MAX_EXPERTS; ++e) {
-      if (e >= E) break;
-      const bf16x8 r =
-          *reinterpret_cast<const bf16x8*>(router + (long)e * K + k);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        acc[e] = fmaf(bits2f(v[j]), bits2f(r[j]), acc[e]);
-    }
-  }
-  __shared__ float red[4][MAX_EXPERTS];
-#pragma unroll
-  for (int e = 0; e < MAX_EXPERTS; ++e) {
-    if (e >= E) break;
-    const float s = wave_sum(acc[e]);
-    if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE][e] = s;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  float logit[MAX_EXPERTS], mx = -INFINITY;
-  for (int e = 0; e < E; ++e) {
-    logit[e] = red[0][e] + red[1][e] + red[2][e] + red[3][e];
-    mx = fmaxf(mx, logit[e]);
-  }
-  // the softmax's denominator cancels in the renormalized weights
-  unsigned taken = 0;
-  float sum = 0.f;
-  for (int i = 0; i < top_k; ++i) {
-    int best = -1;
-    for (int e = 0; e < E; ++e)
-      if (!(taken >> e & 1) && (best < 0 || logit[e] > logit[best])) best = e;
-    taken |= 1u << best;
-    choice[row * top_k + i] = best;
-    const float p = __expf(logit[best] - mx);
-    weight[row * top_k + i] = p;
-    sum += p;
-  }
-  for (int i = 0; i < top_k; ++i) weight[row * top_k + i] /= sum;
-}
-
-}  // namespace
-
 void route_packed(torch::Tensor choice, torch::Tensor weight, torch::Tensor x,
                   torch::Tensor router) {
   const int T = choice.size(0), top_k = choice.size(1);
@@ -777,7 +717,7 @@ void route_packed(torch::Tensor choice, torch::Tensor weight, torch::Tensor x,
   TORCH_CHECK(x.is_contiguous() && x.scalar_type() == at::kBFloat16 &&
               x.numel() == (long)groups * 16 * K);
   if (T == 0) return;
-  hipLaunchKernelGGL(route_packed_kernel, dim3(T), dim3(256), 0,
+  hipLaunchKernelGGL(route_kernel<true>, dim3(T), dim3(256), 0,
                      at::hip::getCurrentHIPStream(), choice.data_ptr<int>(),
                      weight.data_ptr<float>(), (const short*)x.data_ptr(),
                      (const short*)router.data_ptr(), K, groups, E, top_k);
