@@ -36,15 +36,19 @@
 // merged by the workgroup that finishes last, told by a counter per (sequence,
 // kv head) that a kernel earlier in the stream has cleared.
 //
-// The pool is read with non-temporal loads: a layer's cache is not seen again
-// until the next step (48 x 4800 tokens: 184 -> 165 us).
+// The pool is read with non-temporal loads: a layer's cache is mostly not seen
+// again until the next step (48 x 4800 tokens: 188 -> 168 us, 64 x 1100: 61 ->
+// 56). Pages of a prefix that the sequences share are, and the hint costs there,
+// but less: 4096 of 4800 tokens shared by 48 sequences 72.6 -> 74.1 us, 1024 of
+// 1100 by 64 28.7 -> 28.3, by 250 66.0 -> 70.2.
 //
-// Measured (32 heads on 8, page 16, tables of 512 pages, cold cache), against
-// one-wave workgroups that scored with dot instructions, summed V on the VALU
-// and merged 8 fixed splits in a second kernel:
-//   1 x 320 tokens       6 us (14 + 5)      64 x 290       15 us (25 + 5)
-//   13 x 1500, fp8      16 us (49 + 5)      48 x 4800     160 us, 5.9 TB/s (287 + 7)
-//   250 x 600, fp8      56 us (112 + 8)     16 x 1300, 64 heads  23 us (75 + 5)
+// Measured (32 heads on 8, page 16, tables of 512 pages, cold cache, the op
+// with the clearing of its counters), against one-wave workgroups that score
+// with dot instructions, sum V on the VALU and merge 8 fixed splits in a second
+// kernel (decode_attn_fixed.hip):
+//   1 x 320 tokens     9.1 us (14.5)     64 x 290     18.8 us (30.0)
+//   13 x 1500, fp8    18.7 us (50.6)     48 x 4800     168 us, 5.6 TB/s (253)
+//   250 x 600, fp8    59.7 us (111)      16 x 1300, 64 heads  26.1 us (79)
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -431,8 +435,8 @@ int splits_of(long pairs, long max_tokens) {
   // Enough runs for the longest sequence the table can hold, up to a grid of
   // CAP. Workgroups past a sequence's end leave at once but take a slot for
   // a microsecond; the runs are the grid's slowest dimension so that they
-  // come after the ones that work (64 x 290 tokens: 15 us, 31 us with the
-  // runs inside the sequences). Caps of 1024 and 4096 measured 0 to 17 %
+  // come after the ones that work (64 x 290 tokens, with two parts of a
+  // probability: 15 us, 31 us with the runs inside the sequences). Caps of 1024 and 4096 measured 0 to 17 %
   // slower at 250 sequences and within 4 % elsewhere.
   const long want = (max_tokens + chunk_of(pairs) - 1) / chunk_of(pairs);
   return (int)std::max<long>(

@@ -8,9 +8,9 @@
 // four layers of 4-bit experts 0.13, relative 2-norm) without either being
 // nearer to the exact value. Here the order does not depend on the batch or
 // the page table, and a model's outputs stay the bits they have been.
-// decode_attn.hip is the faster one where nothing is quantized behind it: 16
-// against 49 us a layer for 13 x 1500 tokens of fp8 cache, 15 against 25 for
-// 64 x 290 of bf16.
+// decode_attn.hip is the faster one where nothing is quantized behind it: 19
+// against 51 us for 13 x 1500 tokens of fp8 cache, 19 against 30 for 64 x 290 of
+// bf16 (the whole ops, launches included).
 //
 // HBM-bound: streams seq_len * 2 * D values of K/V per (sequence, kv head)
 // once; the GQA group's `ratio` query heads share every value loaded.

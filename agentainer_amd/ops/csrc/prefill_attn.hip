@@ -31,8 +31,8 @@
 //
 // Measured (32 heads on 8, bf16 cache), against the 16x16 tiles of 32 tokens
 // with probabilities going through LDS that were here before: one prompt of
-// 7900 tokens 626 us, 0.82 PFLOP/s (5193 us); 32 prompts of 256 62 us (364);
-// 45 rows over 1245 tokens 10.5 us + 6.1 us merge (198).
+// 7900 tokens 620 us, 0.82 PFLOP/s (5193 us); 32 prompts of 256 63 us (364);
+// 45 rows over 1245 tokens 10.3 us + 5.8 us merge (198).
 //
 // LDS: K keeps the pool's order [16-token group][d/8][16 tokens][8], whose
 // fragment reads are 256 contiguous bytes per 16 lanes; V rows are padded to

@@ -331,7 +331,9 @@ void dispatch_grouped(const StreamArgs& a, const Weights<true>& w, int mode,
 //   8192 x 28672          94 (200)   8192 x 8192        32 (48)
 // A projection that is neither split nor large (qkv: 48 workgroups, 52 us
 // against 26) is left to the library (ops.streams has the line), and so are
-// more than 128 rows, where twice the x makes gate_up 81 us against 70.
+// more than 128 rows, where twice the x makes gate_up 81 us against 70. Two
+// passes of 125 rows lose as well: gate_up 130 us against 88 with the library's
+// silu, qkv 104 against 28, o 28 against 23, down 70 against 63.
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(
     void* __restrict__ out, const char* __restrict__ x,
